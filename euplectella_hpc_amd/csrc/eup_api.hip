@@ -501,10 +501,9 @@ static int ready(eup_handle *h, const char *who)
 
 static int do_steps(eup_handle *h, int32_t nsteps)
 {
+    if (h->cfg.mode == EUP_MODE_PHYSICS) return physics_steps(h, nsteps);
     for (int32_t t = 0; t < nsteps; ++t) {
-        int rc = h->cfg.mode == EUP_MODE_PARITY ? parity_step(h)
-                 : h->cfg.mode == EUP_MODE_GREY ? grey_step(h)
-                                                : physics_step(h);
+        int rc = h->cfg.mode == EUP_MODE_PARITY ? parity_step(h) : grey_step(h);
         if (rc) return rc;
     }
     return 0;

@@ -84,7 +84,7 @@ int parity_step(Handle *h);
 
 // physics mode (eup_physics.hip)
 int physics_prepare_mask(Handle *h);
-int physics_step(Handle *h);
+int physics_steps(Handle *h, int nsteps);
 int physics_refresh_outlet(Handle *h);
 int physics_set_pop(Handle *h, int q); // staging (ghosted f64) -> both buffers
 int physics_get_pop(Handle *h, int q); // current buffer -> staging

@@ -1,4 +1,4 @@
-// Physics mode: fused pull collide+stream, one launch per time step.
+// Physics mode: fused pull collide+stream, one launch per time step, or one per two (eup_pair.h).
 //
 // The step has the arithmetic of the reference's col.F90:127-229 and the inlet/outlet formulas of
 // bcond.bc.F90, with the y/z periodicity applied by index wrap (ghosts always fresh, so there is
@@ -26,6 +26,7 @@
 // read one step later, so no extra pass over the lattice is needed.
 #include <stdlib.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "eup_internal.h"
@@ -469,6 +470,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(1, 3))) 
     fused_step<double, true>(a);
 }
 
+#include "eup_pair.h"
+
 // ---------------------------------------------------------------------------------------------
 // mask preparation
 // ---------------------------------------------------------------------------------------------
@@ -514,6 +517,11 @@ __global__ __launch_bounds__(kBlock) void k_classify(const uint8_t *__restrict__
     else c = 1;
     if ((threadIdx.x & 63) == 0) cls[t] = c;
     link_all[(size_t)t * kTile + (threadIdx.x & 63)] = lm;
+}
+
+__global__ void k_uniform_links(uint32_t *__restrict__ link)
+{
+    link[threadIdx.x] = threadIdx.x < kTile ? 0u : 0x80000000u;
 }
 
 __global__ void k_compact_links(const int32_t *__restrict__ code, const uint32_t *__restrict__ link_all,
@@ -775,6 +783,79 @@ template <typename S> int step_t(Handle *h)
     return 0;
 }
 
+// The two-step kernel's cut of the lattice and, in us, the time that a pair is expected to take:
+// zc planes per chunk in the number of rounds that the workgroups need (one per CU) cost a run-up
+// and t1 per plane.  Of cuts that are equal within 4 % the one with the most chunks is taken, which
+// evens out the columns with obstacles (192 x 768 x 768 sponge FP32: 1.88 ms per step with 24 chunks of
+// 32 planes, 2.01 with 7 of 110).
+template <typename S> PairMap pair_map(const Handle *h, double *us)
+{
+    using Sh = PairShape<S>;
+    // measured on MI355X: 128 x 64 x 64 (1 round of 3 planes) 29 us, 256 x 128 x 128 (22) 163 us in
+    // FP32; 64 x 64 x 64 (1 round of 4) 38 us, 128 x 128 x 128 (26) 193 us in FP64
+    constexpr double t0 = sizeof(S) == 4 ? 8.0 : 11.0, t1 = sizeof(S) == 4 ? 6.4 : 7.0;
+    const Geometry &g = h->g;
+    PairMap pm;
+    pm.nx = (uint32_t)((g.l + Sh::tx - 1) / Sh::tx);
+    pm.ny = (uint32_t)((g.m + Sh::ty - 1) / Sh::ty);
+    int cus = 0;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, h->cfg.device) != hipSuccess || cus <= 0)
+        cus = 256;
+    const int64_t cols = (int64_t)pm.nx * pm.ny;
+    double best = 1e300;
+    pm.zc = 1;
+    for (int nz = 1; nz <= g.n; ++nz) {
+        const int zc = (g.n + nz - 1) / nz;
+        const int64_t blocks = cols * ((g.n + zc - 1) / zc);
+        const double c = (double)((blocks + cus - 1) / cus) * (t0 + t1 * zc);
+        if (c <= 1.04 * best) pm.zc = (uint32_t)zc;
+        best = std::min(best, c);
+    }
+    if (const char *e = getenv("EUP_PAIR_ZC")) pm.zc = (uint32_t)atoi(e);
+    pm.blocks = (uint32_t)(cols * ((g.n + (int)pm.zc - 1) / (int)pm.zc));
+    pm.dnx = UDiv::make(pm.nx);
+    pm.dny = UDiv::make(pm.ny);
+    pm.plane = (uint32_t)((uint64_t)g.tiles_per_row * (uint64_t)g.m * kTileElems * sizeof(S));
+    pm.mixed = (int)h->tiles_mixed;
+    *us = best;
+    return pm;
+}
+
+// Whether the handle's steps are taken two per launch: where a pair is expected to be at least a tenth
+// faster than two single steps (columns with obstacles cost a pair up to that much more), these at the
+// 6.1 TB/s and 2.5 us per launch that they reach.  Measured, single against pair per step, without
+// obstacles: FP32 64 x 64 x 64 8.5 / 10.1 us (single), 128 x 64 x 64 16.2 / 14.6, 256 x 128 x 128
+// 105 / 82, 680 x 340 x 4 27.3 / 30.8 (single), 512 x 256 x 256 813 / 571; FP64 128 x 64 x 64 30.3 / 30.5
+// (single), 256 x 128 x 128 210 / 178, 512 x 256 x 256 1659 / 1285.
+template <typename S> bool pair_better(const Handle *h)
+{
+    const Geometry &g = h->g;
+    // offsets within a plane of tiles and within the outlet planes stay below 2^31
+    const uint64_t plane = (uint64_t)g.tiles_per_row * (uint64_t)g.m * kTileElems * sizeof(S);
+    if (plane >= (1ull << 31) || (uint64_t)g.m * g.n * 5 * sizeof(S) >= (1ull << 31)) return false;
+    if (const char *e = getenv("EUP_PAIR")) return atoi(e) != 0;
+    double us;
+    pair_map<S>(h, &us);
+    return 1.1 * us < 2.0 * (2.5 + (double)g.tiles * (2 * kTileElems * sizeof(S)) / 6.1e6);
+}
+
+template <typename S, bool XOPEN> int pair_launches(Handle *h, int count)
+{
+    const size_t lds = pair_lds_bytes<S>();
+    if (hip_check(h, hipFuncSetAttribute(reinterpret_cast<const void *>(k_pair<S, XOPEN>),
+                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds), "two-step LDS"))
+        return EUP_EHIP;
+    double us;
+    const PairMap pm = pair_map<S>(h, &us);
+    for (int i = 0; i < count; ++i) {
+        const XArgs<S> a = make_args<S>(h);
+        hipLaunchKernelGGL((k_pair<S, XOPEN>), dim3(pm.blocks), dim3(pair_threads<S>()), lds, h->stream, a, pm);
+        if (hip_check(h, hipGetLastError(), "two-step launch")) return EUP_EHIP;
+        h->cur ^= 1;
+    }
+    return 0;
+}
+
 template <typename S> int refresh_t(Handle *h)
 {
     using R = typename Store<S>::compute;
@@ -820,13 +901,24 @@ template <typename F> int dispatch(Handle *h, F &&f)
 
 } // namespace
 
-int physics_step(Handle *h)
+int physics_steps(Handle *h, int nsteps)
 {
-    if (h->outlet_dirty) {
+    if (nsteps > 0 && h->outlet_dirty) {
         int rc = physics_refresh_outlet(h);
         if (rc) return rc;
     }
-    return dispatch(h, [&](auto *p) { return step_t<std::remove_pointer_t<decltype(p)>>(h); });
+    return dispatch(h, [&](auto *p) -> int {
+        using S = std::remove_pointer_t<decltype(p)>;
+        int t = 0, rc = 0;
+        if constexpr (kPairs<S>) {
+            if (nsteps > 1 && pair_better<S>(h)) {
+                rc = x_open(h) ? pair_launches<S, true>(h, nsteps / 2) : pair_launches<S, false>(h, nsteps / 2);
+                t = nsteps / 2 * 2;
+            }
+        }
+        for (; t < nsteps && !rc; ++t) rc = step_t<S>(h);
+        return rc;
+    });
 }
 
 int physics_refresh_outlet(Handle *h)
@@ -905,11 +997,16 @@ int physics_prepare_mask(Handle *h)
         h->tile_code = nullptr;
         h->link_mask = nullptr;
         if (hip_check(h, hipMalloc((void **)&h->tile_code, sizeof(int32_t) * g.tiles), "hipMalloc") ||
-            hip_check(h, hipMalloc((void **)&h->link_mask, sizeof(uint32_t) * kTile * (nm > 0 ? nm : 1)),
+            hip_check(h, hipMalloc((void **)&h->link_mask, sizeof(uint32_t) * kTile * (nm + 2)),
                       "hipMalloc") ||
             hip_check(h, hipMemcpyAsync(h->tile_code, code_h, sizeof(int32_t) * g.tiles,
                                         hipMemcpyHostToDevice, h->stream), "copy"))
             rc = EUP_EHIP;
+    }
+    if (!rc) {
+        // the masks of a fluid and of a solid tile after the mixed tiles' (two-step kernel)
+        hipLaunchKernelGGL(k_uniform_links, dim3(1), dim3(2 * kTile), 0, h->stream, h->link_mask + nm * kTile);
+        if (hip_check(h, hipGetLastError(), "uniform links")) rc = EUP_EHIP;
     }
     if (!rc && nm > 0) {
         hipLaunchKernelGGL(k_compact_links, dim3(grid), dim3(kBlock), 0, h->stream, h->tile_code,

@@ -1,0 +1,57 @@
+"""Two steps per launch (FP32 and FP64 physics mode) against one step per launch: the same state, outlet
+plane and drag, bit for bit, on lattices at the edges of the two-step kernel's windows (FP32 64 x 13
+sites, FP64 32 x 12) and chunks.  The environment switch EUP_PAIR forces either form, so that sizes
+for which single steps are the faster choice are covered too."""
+import numpy as np
+import pytest
+
+from euplectella_hpc_amd import geometry
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(2, 2, 2), (33, 2, 4), (34, 30, 3), (63, 13, 5), (64, 12, 7), (65, 14, 9), (70, 45, 36), (130, 27, 6),
+          (192, 25, 11)]
+
+
+def after(shape, storage, x_open, mask, steps, pair, monkeypatch):
+    from euplectella_hpc_amd.lib import Lattice
+
+    monkeypatch.setenv("EUP_PAIR", pair)
+    with Lattice(*shape, svisc=0.05, u_inflow=0.05, mode="physics", storage=storage, x_open=x_open,
+                 fgrad=0.0 if x_open else 1e-5) as lat:
+        lat.set_mask(mask)
+        lat.init_equilibrium(0.05, 0.01, -0.02, 1e-2, 3)
+        lat.step(steps)
+        state, drag = lat.get_state(), lat.drag_mem()
+        monkeypatch.setenv("EUP_PAIR", "0")
+        lat.step(1)  # a further single step reads the outlet plane that the last one left
+        return state, drag, lat.get_state()
+
+
+@pytest.mark.parametrize("storage", ["f32", "f64"])
+@pytest.mark.parametrize("x_open", [True, False])
+@pytest.mark.parametrize("shape", SHAPES)
+def test_two_steps_equal_single_steps(shape, x_open, storage, monkeypatch):
+    print(f"two-step {shape} x_open={x_open} {storage}", flush=True)
+    # solid sites everywhere, the first and last x planes and the periodic seams included
+    mask = geometry.scattered(*shape, fraction=0.08, seed=5)
+    for steps in (2, 5):
+        one = after(shape, storage, x_open, mask, steps, "0", monkeypatch)
+        two = after(shape, storage, x_open, mask, steps, "1", monkeypatch)
+        for a, b in zip(one, two):
+            assert np.isfinite(a).all()
+            assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("storage", ["f32", "f64"])
+@pytest.mark.parametrize("chunk", ["1", "3", "7"])
+def test_chunks_of_planes(chunk, storage, monkeypatch):
+    """Any cut into chunks of planes gives the same state, the last chunk a short one."""
+    shape = (100, 20, 17)
+    print(f"two-step chunks of {chunk} planes {storage}", flush=True)
+    mask = geometry.cylinder(*shape, 5, (25, 10))
+    one = after(shape, storage, True, mask, 4, "0", monkeypatch)
+    monkeypatch.setenv("EUP_PAIR_ZC", chunk)
+    two = after(shape, storage, True, mask, 4, "1", monkeypatch)
+    for a, b in zip(one, two):
+        assert np.array_equal(a, b)
