@@ -111,7 +111,7 @@ static void release(Handle *h)
     if (h->stream) hipStreamSynchronize(h->stream);
     void *ptrs[] = {h->alloc[0], h->alloc[1], h->staging, h->obs_stage, h->solid, h->solid_list, h->bb_tmp,
                     h->tile_code, h->link_mask, h->mixed_list, h->outlet[0], h->outlet[1], h->diag,
-                    h->site19, h->grey};
+                    h->site19, h->grey, h->grey_zero, h->work};
     for (void *p : ptrs)
         if (p) hipFree(p);
     if (h->ev0) hipEventDestroy(h->ev0);
@@ -232,7 +232,8 @@ int eup_create(const eup_config *cfg, eup_handle **out)
         rc = EUP_EHIP;
     // physics mode: tile-major with one guard tile on either side; other modes: SoA
     const size_t state = h->tiled ? h->elem * (size_t)kTileElems * (size_t)(g.tiles + 2)
-                                  : h->elem * (size_t)h->stride * 19;
+                                  : cfg->mode == EUP_MODE_GREY ? grey_state_bytes(h)
+                                                               : h->elem * (size_t)h->stride * 19;
     const size_t lead = h->tiled ? h->elem * (size_t)kTileElems : 0;
     for (int b = 0; b < 2 && !rc; ++b) {
         if (hip_check(h, hipMalloc(&h->alloc[b], state), "hipMalloc populations")) rc = EUP_EHIP;

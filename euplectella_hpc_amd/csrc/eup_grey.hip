@@ -18,10 +18,11 @@
 //   lam_p(z) = (1 - sigma_l) lin_p(z + c_p) + sigma_l lin_pbar(z)   (sigma_l of link z -- z + c_p)
 // plus the outlet-equilibrium transpose on the last x column and the objective terms, and adds the
 // gradient terms of the links of which the site is the source (FP64 accumulation).
-// Inside a recomputed segment k_adj_fused (the FP64 default) runs the stream half of step t and the
-// collide half of step t - 1 in one pass, so lam^t is never stored.
-// States are checkpointed every K steps; each segment is recomputed forward and stored before its
-// backward sweep, so memory is (t1/K + K) states instead of t1.
+// Inside a segment k_adj_fused runs the stream half of step t and the collide half of step t - 1 in
+// one pass, so lam^t is never stored.
+// States are checkpointed every K steps; each segment but the last, whose states the forward sweep
+// leaves in place, is recomputed forward before its backward sweep, so memory is (t1/K + K) states
+// instead of t1.
 #include <cstdlib>
 #include <type_traits>
 #include <vector>
@@ -39,145 +40,121 @@ constexpr int kCY[19] = {-1, 0, 1, 0, 0, 0, 1, 1, 1, -1, 0, 1, 0, 0, 0, -1, -1, 
 constexpr int kCZ[19] = {0, -1, 0, 1, 0, 1, 1, 0, -1, 0, -1, 0, 1, 0, -1, -1, 0, 1, 0};
 constexpr int kOPP[19] = {11, 12, 9, 10, 13, 14, 15, 16, 17, 2, 3, 0, 1, 4, 5, 6, 7, 8, 18};
 
-// a state: 19 SoA arrays of l*m*n sites, population q at A + q * stride
+// A state: 19 SoA arrays of l*m*n sites, population q at A + q * stride, then the outlet ghost plane
+// of the state (5 x m x n: the equilibria that bcond.bc.F90:138-164 gives for its x = l column), which
+// the kernel that writes the state writes too.  (Evaluated by each reader instead, an x = l site
+// loaded 19 populations for each of its five outlet links, and every wavefront with such a site
+// waited for it.)
 template <typename R> struct GArgs {
     const R *A; // the state read
     R *B;       // the state written, or null
     int64_t stride;
     const R *s;
+    const uint8_t *zero; // per 64 consecutive sites: s = 0 there and at all their neighbours
+    double *partial;     // three force sums per block
     R inl[5];
     R omega;
     int l, m, n;
     int xopen;
-    __device__ __forceinline__ R a(int q, int64_t x) const { return A[q * stride + x]; }
+    UDiv dl, dm;
 };
 
-struct Nbr {
-    int l, m, n, xopen;
-    // site index of (i + dx, j + dy, k + dz), wrapping y and z (and x when periodic); -1 = inlet
-    // ghost, -2 = outlet ghost
-    __device__ __forceinline__ int64_t at(int i, int j, int k, int dx, int dy, int dz) const
-    {
-        int ii = i + dx, jj = j + dy, kk = k + dz;
-        jj = jj < 0 ? jj + m : (jj >= m ? jj - m : jj);
-        kk = kk < 0 ? kk + n : (kk >= n ? kk - n : kk);
-        if (ii < 0) {
-            if (xopen) return -1;
-            ii += l;
-        } else if (ii >= l) {
-            if (xopen) return -2;
-            ii -= l;
-        }
-        return (int64_t)ii + (int64_t)l * ((int64_t)jj + (int64_t)m * kk);
-    }
+// addresses: element e of an array; 32-bit byte offsets (one scalar base per array, one lane offset)
+// where the array is smaller than 4 GiB, 64-bit ones otherwise
+template <bool BIG, typename R> __device__ __forceinline__ R ldg(const R *p, uint32_t e)
+{
+    if constexpr (BIG) return p[(uint64_t)e];
+    else return *reinterpret_cast<const R *>(reinterpret_cast<const char *>(p) + (uint64_t)(e * (uint32_t)sizeof(R)));
+}
+
+template <bool BIG, typename R> __device__ __forceinline__ void stg(R *p, uint32_t e, R v)
+{
+    if constexpr (BIG) p[(uint64_t)e] = v;
+    else *reinterpret_cast<R *>(reinterpret_cast<char *>(p) + (uint64_t)(e * (uint32_t)sizeof(R))) = v;
+}
+
+// one thread per site: its index, coordinates and the index steps to its neighbours (d = -1, 0, +1 at
+// [d + 1]), wrapped in y and z (and x when periodic; with open x a step past the end stays on the site
+// and the caller takes the ghost instead)
+struct Site {
+    uint32_t x;
+    int i, j, k;
+    uint32_t dx[3], dy[3], dz[3];
+    bool first, last; // open x: the first and the last column
+    bool valid;
+    __device__ __forceinline__ uint32_t at(int cx, int cy, int cz) const { return x + dx[cx + 1] + dy[cy + 1] + dz[cz + 1]; }
+    // open x: the neighbour at +c_x is the inlet or outlet ghost
+    __device__ __forceinline__ bool ghost(int cx) const { return cx == 1 ? last : (cx == -1 && first); }
 };
+
+template <typename R> __device__ __forceinline__ Site site_of(const GArgs<R> &a)
+{
+    Site p;
+    const uint32_t l = (uint32_t)a.l, m = (uint32_t)a.m, n = (uint32_t)a.n, N = l * m * n;
+    p.x = blockIdx.x * blockDim.x + threadIdx.x;
+    p.valid = p.x < N;
+    const uint32_t x = p.valid ? p.x : N - 1, row = a.dl.div(x), k = a.dm.div(row);
+    p.x = x;
+    p.i = (int)(x - row * l);
+    p.j = (int)(row - k * m);
+    p.k = (int)k;
+    p.first = a.xopen && p.i == 0;
+    p.last = a.xopen && p.i == a.l - 1;
+    p.dx[0] = p.i > 0 ? 0u - 1u : (a.xopen ? 0u : l - 1);
+    p.dx[2] = p.i < a.l - 1 ? 1u : (a.xopen ? 0u : 0u - (l - 1));
+    p.dy[0] = p.j > 0 ? 0u - l : (m - 1) * l;
+    p.dy[2] = p.j < a.m - 1 ? l : 0u - (m - 1) * l;
+    const uint32_t lm = l * m;
+    p.dz[0] = p.k > 0 ? 0u - lm : (n - 1) * lm;
+    p.dz[2] = p.k < a.n - 1 ? lm : 0u - (n - 1) * lm;
+    p.dx[1] = p.dy[1] = p.dz[1] = 0u;
+    return p;
+}
 
 template <typename R> __device__ __forceinline__ R wq(int q)
 {
     return q == 18 ? R(1) / R(3) : ((kCX[q] * kCX[q] + kCY[q] * kCY[q] + kCZ[q] * kCZ[q]) == 1 ? R(1) / R(18) : R(1) / R(36));
 }
 
-// link q of site (i,j,k) (0-based): sv the source value, syv the source's solid fraction (0 on a
-// ghost), kd 0 interior, 1 inlet, 2 outlet.  Called inside fully unrolled loops, so q is a
-// compile-time constant.
-template <typename R>
-__device__ __forceinline__ void grey_link(const GArgs<R> &a, const Nbr &nb, int i, int j, int k, int q, R &sv,
-                                          R &syv, int &kd)
+// whether the wavefront's sites are free fluid with free neighbours (s = 0: every link sigma is zero)
+template <typename R> __device__ __forceinline__ bool chunk_zero(const GArgs<R> &a, const Site &p)
 {
-    const int64_t y = nb.at(i, j, k, -kCX[q], -kCY[q], -kCZ[q]);
-    if (kCX[q] == 1 && y == -1) { // only c_x = +1 pulls from the inlet ghost
-        sv = a.inl[kCX[q] == 1 ? q : 0];
-        syv = R(0);
-        kd = 1;
-    } else if (kCX[q] == -1 && y == -2) { // only c_x = -1 pulls from the outlet ghost
-        const int64_t z = nb.at(a.l - 1, j, k, 0, -kCY[q], -kCZ[q]);
-        R yv[19], o[5];
+    return a.zero[__builtin_amdgcn_readfirstlane(p.x >> 6)] != 0;
+}
+
+// outlet ghost values that the last column pulls as populations 9..13: entry (j - c_y, k - c_z)
+template <typename R> __device__ __forceinline__ void outlet_pulls(const GArgs<R> &a, const Site &p, R *src)
+{
+    const R *out = a.A + 19 * a.stride;
+    const uint32_t mn = (uint32_t)a.m * (uint32_t)a.n;
+    const uint32_t jm = p.j > 0 ? p.j - 1 : a.m - 1, jp = p.j < a.m - 1 ? p.j + 1 : 0;
+    const uint32_t km = p.k > 0 ? p.k - 1 : a.n - 1, kp = p.k < a.n - 1 ? p.k + 1 : 0;
 #pragma unroll
-        for (int p = 0; p < 19; ++p) yv[p] = a.a(p, z);
-        outlet_eq<R>(yv, o);
-        sv = o[kCX[q] == -1 ? q - 9 : 0];
-        syv = R(0);
-        kd = 2;
-    } else {
-        sv = a.a(q, y);
-        syv = a.s[y];
-        kd = 0;
+    for (int q = 9; q < 14; ++q) {
+        const uint32_t jj = kCY[q] == 0 ? (uint32_t)p.j : (kCY[q] > 0 ? jm : jp);
+        const uint32_t kk = kCZ[q] == 0 ? (uint32_t)p.k : (kCZ[q] > 0 ? km : kp);
+        src[q] = out[(uint32_t)(q - 9) * mn + jj + (uint32_t)a.m * kk];
     }
 }
 
-// pulled populations f[19] of site (i,j,k) (0-based): per link sigma = 1 - (1 - s(x))(1 - s(y))
-// and f_q = (1 - sigma) src_q + sigma a_qbar(x)
-template <typename R>
-__device__ __forceinline__ void grey_pull(const GArgs<R> &a, const Nbr &nb, int i, int j, int k, int64_t x, R *f)
+// source values src[0..17] that site p pulls (population 18 stays): interior sources, the inlet
+// equilibrium, the outlet ghost plane
+template <bool BIG, typename R> __device__ __forceinline__ void sources(const GArgs<R> &a, const Site &p, R *src)
 {
-    const R sx = a.s[x];
 #pragma unroll
-    for (int q = 0; q < 18; ++q) {
-        R sv, syv;
-        int kd;
-        grey_link<R>(a, nb, i, j, k, q, sv, syv, kd);
-        const R sg = R(1) - (R(1) - sx) * (R(1) - syv);
-        f[q] = (R(1) - sg) * sv + sg * a.a(kOPP[q], x);
+    for (int q = 0; q < 18; ++q) src[q] = ldg<BIG>(a.A + q * a.stride, p.at(-kCX[q], -kCY[q], -kCZ[q]));
+    if (p.first) {
+#pragma unroll
+        for (int q = 0; q < 5; ++q) src[q] = a.inl[q];
     }
-    f[18] = a.a(18, x);
+    if (p.last) outlet_pulls(a, p, src);
 }
 
-// grey_pull that also returns the links: sig[q] the link fraction, src[q] the source value,
-// sy[q] the source's solid fraction (0 on a ghost), kind[q] 0 interior, 1 inlet, 2 outlet.  The
-// same arithmetic as grey_link + grey_pull, written out: the FP32 adjoint collide built on it
-// takes 166 registers per lane, built on grey_link 186 (three against two wavefronts per SIMD).
-template <typename R>
-__device__ __forceinline__ void grey_pull_links(const GArgs<R> &a, const Nbr &nb, int i, int j, int k, int64_t x, R *f,
-                                          R *sig, R *src, R *sy, int *kind)
+// solid fraction of the source of population q (0 on the ghosts)
+template <bool BIG, typename R> __device__ __forceinline__ R source_s(const GArgs<R> &a, const Site &p, int q)
 {
-    const R sx = a.s[x];
-#pragma unroll
-    for (int q = 0; q < 18; ++q) {
-        const int64_t y = nb.at(i, j, k, -kCX[q], -kCY[q], -kCZ[q]);
-        R sv, syv;
-        int kd;
-        if (kCX[q] == 1 && y == -1) { // only c_x = +1 pulls from the inlet ghost
-            sv = a.inl[kCX[q] == 1 ? q : 0];
-            syv = R(0);
-            kd = 1;
-        } else if (kCX[q] == -1 && y == -2) { // only c_x = -1 pulls from the outlet ghost
-            const int64_t z = nb.at(a.l - 1, j, k, 0, -kCY[q], -kCZ[q]);
-            R yv[19], o[5];
-#pragma unroll
-            for (int p = 0; p < 19; ++p) yv[p] = a.a(p, z);
-            outlet_eq<R>(yv, o);
-            sv = o[kCX[q] == -1 ? q - 9 : 0];
-            syv = R(0);
-            kd = 2;
-        } else {
-            sv = a.a(q, y);
-            syv = a.s[y];
-            kd = 0;
-        }
-        const R sg = R(1) - (R(1) - sx) * (R(1) - syv);
-        sig[q] = sg;
-        src[q] = sv;
-        sy[q] = syv;
-        kind[q] = kd;
-        f[q] = (R(1) - sg) * sv + sg * a.a(kOPP[q], x);
-    }
-    f[18] = a.a(18, x);
-}
-
-template <typename R> __global__ __launch_bounds__(256) void k_grey_step(GArgs<R> a)
-{
-    const int64_t x = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t N = (int64_t)a.l * a.m * a.n;
-    if (x >= N) return;
-    const int i = (int)(x % a.l);
-    const int64_t r = x / a.l;
-    const int j = (int)(r % a.m), k = (int)(r / a.m);
-    Nbr nb{a.l, a.m, a.n, a.xopen};
-    R f[19];
-    grey_pull<R>(a, nb, i, j, k, x, f);
-    collide<R>(f, f, a.omega, R(0));
-#pragma unroll
-    for (int q = 0; q < 19; ++q) a.B[q * a.stride + x] = f[q];
+    const R v = ldg<BIG>(a.s, p.at(-kCX[q], -kCY[q], -kCZ[q]));
+    return p.ghost(-kCX[q]) ? R(0) : v;
 }
 
 __device__ __forceinline__ double wsum(double v)
@@ -186,45 +163,90 @@ __device__ __forceinline__ double wsum(double v)
     return v;
 }
 
-// block partial sums of the force (3 doubles per block)
-template <typename R> __global__ __launch_bounds__(256) void k_grey_force(GArgs<R> a, double *partial)
+// partial[3 * block ..] += the block's sums of the first NF components of v (one block is always the
+// same sites, so the sums over sites and steps have a fixed order)
+template <int NF> __device__ __forceinline__ void add_partial(const double *v, double *partial)
 {
-    const int64_t N = (int64_t)a.l * a.m * a.n;
-    Nbr nb{a.l, a.m, a.n, a.xopen};
-    double v[3] = {0.0, 0.0, 0.0};
-    for (int64_t x = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; x < N; x += (int64_t)gridDim.x * blockDim.x) {
-        const int i = (int)(x % a.l);
-        const int64_t r = x / a.l;
-        const int j = (int)(r % a.m), k = (int)(r / a.m);
-        const R sx = a.s[x];
-#pragma unroll
-        for (int q = 0; q < 18; ++q) {
-            R sv, syv;
-            int kd;
-            grey_link<R>(a, nb, i, j, k, q, sv, syv, kd);
-            if (kd != 0) continue;
-            const R sg = R(1) - (R(1) - sx) * (R(1) - syv);
-            const double d = (double)sg * ((double)sv - (double)a.a(kOPP[q], x));
-            v[0] += kCX[q] * d;
-            v[1] += kCY[q] * d;
-            v[2] += kCZ[q] * d;
-        }
-    }
-    __shared__ double sh[3][4];
+    __shared__ double sh[NF][4];
     const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    for (int c = 0; c < 3; ++c) {
-        double t = wsum(v[c]);
+    for (int c = 0; c < NF; ++c) {
+        const double t = wsum(v[c]);
         if (lane == 0) sh[c][w] = t;
     }
     __syncthreads();
-    if (threadIdx.x == 0)
-        for (int c = 0; c < 3; ++c) partial[blockIdx.x * 3 + c] = sh[c][0] + sh[c][1] + sh[c][2] + sh[c][3];
+    if (threadIdx.x < NF)
+        partial[blockIdx.x * 3 + threadIdx.x] += sh[threadIdx.x][0] + sh[threadIdx.x][1] + sh[threadIdx.x][2] + sh[threadIdx.x][3];
 }
 
-// acc[c] += weight * sum of partials (single block, fixed order)
-__global__ void k_force_acc(const double *partial, int nb, double weight, double *acc, double *last)
+// One step of the grey lattice and the force of the state read, its first NF components (both pull the
+// same links).  Without STEP only the force.  Memory-bound: 19 reads and 19 writes per site, and 18 + 18
+// more reads, of own populations and solid fractions, that mostly hit the caches and that wavefronts
+// of free fluid skip.  128 x 64 x 64 FP32: 18.1 us (23.3 with 64-bit index arithmetic, every outlet
+// value evaluated where it is read and no chunk flags), 21.8 with the force (it took 17.6 + 4.6 us on
+// its own); FP64 70 x 45 x 36 10.9 us (15.4).
+template <typename R, bool BIG, bool STEP, int NF> __global__ __launch_bounds__(256) void k_grey(GArgs<R> a)
 {
-    __shared__ double sh[3][256];
+    const Site p = site_of(a);
+    const bool zero = chunk_zero(a, p);
+    double v[3] = {0.0, 0.0, 0.0};
+    if (STEP || !zero) {
+        R f[19];
+        sources<BIG>(a, p, f);
+        f[18] = ldg<BIG>(a.A + 18 * a.stride, p.x);
+        if (!zero) {
+            const R sx = ldg<BIG>(a.s, p.x);
+            R own[18];
+#pragma unroll
+            for (int q = 0; q < 18; ++q) own[q] = ldg<BIG>(a.A + kOPP[q] * a.stride, p.x);
+#pragma unroll
+            for (int q = 0; q < 18; ++q) {
+                const R sg = R(1) - (R(1) - sx) * (R(1) - source_s<BIG>(a, p, q));
+                if (NF > 1 || (NF == 1 && kCX[q])) {
+                    const double d = p.valid && !p.ghost(-kCX[q]) ? (double)sg * ((double)f[q] - (double)own[q]) : 0.0;
+                    if (kCX[q]) v[0] += kCX[q] * d;
+                    if (NF > 1 && kCY[q]) v[1] += kCY[q] * d;
+                    if (NF > 1 && kCZ[q]) v[2] += kCZ[q] * d;
+                }
+                f[q] = (R(1) - sg) * f[q] + sg * own[q];
+            }
+        }
+        if constexpr (STEP) {
+            collide<R>(f, f, a.omega, R(0));
+            if (p.valid) {
+#pragma unroll
+                for (int q = 0; q < 19; ++q) stg<BIG>(a.B + q * a.stride, p.x, f[q]);
+                if (p.last) {
+                    R o[5];
+                    outlet_eq<R>(f, o);
+                    const uint32_t mn = (uint32_t)a.m * (uint32_t)a.n;
+#pragma unroll
+                    for (uint32_t u = 0; u < 5; ++u) a.B[19 * a.stride + u * mn + p.j + (uint32_t)a.m * (uint32_t)p.k] = o[u];
+                }
+            }
+        }
+    }
+    if constexpr (NF > 0) {
+        if (__syncthreads_or(!zero)) add_partial<NF>(v, a.partial);
+    }
+}
+
+// outlet ghost plane of a state that the host set
+template <typename R> __global__ __launch_bounds__(256) void k_grey_outlet(R *A, int64_t stride, int l, int m, int n)
+{
+    const uint32_t r = blockIdx.x * blockDim.x + threadIdx.x, mn = (uint32_t)m * (uint32_t)n;
+    if (r >= mn) return;
+    R y[19], o[5];
+#pragma unroll
+    for (int q = 0; q < 19; ++q) y[q] = A[q * stride + (int64_t)r * l + l - 1];
+    outlet_eq<R>(y, o);
+#pragma unroll
+    for (uint32_t u = 0; u < 5; ++u) A[19 * stride + u * mn + r] = o[u];
+}
+
+// the sums of the blocks' partial forces (single block, fixed order)
+__global__ __launch_bounds__(1024) void k_force_sum(const double *partial, int nb, double *out)
+{
+    __shared__ double sh[3][1024];
     double v[3] = {0.0, 0.0, 0.0};
     for (int b = threadIdx.x; b < nb; b += blockDim.x)
         for (int c = 0; c < 3; ++c) v[c] += partial[b * 3 + c];
@@ -235,39 +257,46 @@ __global__ void k_force_acc(const double *partial, int nb, double weight, double
             for (int c = 0; c < 3; ++c) sh[c][threadIdx.x] += sh[c][threadIdx.x + st];
         __syncthreads();
     }
-    if (threadIdx.x == 0)
-        for (int c = 0; c < 3; ++c) {
-            last[c] = sh[c][0];
-            acc[c] += weight * sh[c][0];
-        }
+    if (threadIdx.x < 3) out[threadIdx.x] = sh[threadIdx.x][0];
 }
 
-// transposed BGK Jacobian at pre-collision f applied to lam
-template <typename R> __device__ __forceinline__ void collide_adj(const R *f, const R *lam, R omega, R *out)
+// Transposed BGK Jacobian at density rho and momentum j applied to lam[19], in place:
+//   out_p = (1 - omega) lam_p + omega (A + B . c_p),
+//   A = sum_q lam_q w_q (1 + 1.5 u^2 - 4.5 (c_q.u)^2),
+//   B = sum_q lam_q w_q (3 c_q + 9 (c_q.u) c_q - 3 u).
+// Only the terms with c != 0 are formed (a product with a constant 0 is not dropped by the compiler).
+template <typename R> __device__ __forceinline__ void collide_adj(R rho, R jx, R jy, R jz, R omega, R *lam)
 {
-    R rho = 0, jx = 0, jy = 0, jz = 0;
+    const R inv = R(1) / rho, ux = jx * inv, uy = jy * inv, uz = jz * inv, usq = ux * ux + uy * uy + uz * uz;
+    R S = 0, Q = 0, Bx = 0, By = 0, Bz = 0;
 #pragma unroll
     for (int q = 0; q < 19; ++q) {
-        rho += f[q];
-        jx += kCX[q] * f[q];
-        jy += kCY[q] * f[q];
-        jz += kCZ[q] * f[q];
+        const R lw = lam[q] * wq<R>(q);
+        S += lw;
+        if (q == 18) continue;
+        R cu = R(0);
+        if (kCX[q]) cu = kCX[q] > 0 ? ux : -ux;
+        if (kCY[q]) cu = kCY[q] > 0 ? cu + uy : cu - uy;
+        if (kCZ[q]) cu = kCZ[q] > 0 ? cu + uz : cu - uz;
+        Q += lw * (cu * cu);
+        const R g = lw * (R(3) + R(9) * cu);
+        if (kCX[q]) Bx = kCX[q] > 0 ? Bx + g : Bx - g;
+        if (kCY[q]) By = kCY[q] > 0 ? By + g : By - g;
+        if (kCZ[q]) Bz = kCZ[q] > 0 ? Bz + g : Bz - g;
     }
-    const R ux = jx / rho, uy = jy / rho, uz = jz / rho, usq = ux * ux + uy * uy + uz * uz;
-    R A = 0, Bx = 0, By = 0, Bz = 0;
+    const R A = S * (R(1) + R(1.5) * usq) - R(4.5) * Q, S3 = R(3) * S;
+    Bx -= S3 * ux;
+    By -= S3 * uy;
+    Bz -= S3 * uz;
+    const R o1 = R(1) - omega;
 #pragma unroll
-    for (int q = 0; q < 19; ++q) {
-        const R w = wq<R>(q);
-        const R cu = kCX[q] * ux + kCY[q] * uy + kCZ[q] * uz;
-        A += lam[q] * w * (R(1) - R(4.5) * cu * cu + R(1.5) * usq);
-        const R g = lam[q] * w * (R(3) + R(9) * cu);
-        Bx += g * kCX[q] - lam[q] * w * R(3) * ux;
-        By += g * kCY[q] - lam[q] * w * R(3) * uy;
-        Bz += g * kCZ[q] - lam[q] * w * R(3) * uz;
+    for (int p = 0; p < 19; ++p) {
+        R e = A;
+        if (kCX[p]) e = kCX[p] > 0 ? e + Bx : e - Bx;
+        if (kCY[p]) e = kCY[p] > 0 ? e + By : e - By;
+        if (kCZ[p]) e = kCZ[p] > 0 ? e + Bz : e - Bz;
+        lam[p] = o1 * lam[p] + omega * e;
     }
-#pragma unroll
-    for (int p = 0; p < 19; ++p)
-        out[p] = (R(1) - omega) * lam[p] + omega * (A + Bx * kCX[p] + By * kCY[p] + Bz * kCZ[p]);
 }
 
 template <typename R> struct AdjArgs {
@@ -281,261 +310,227 @@ template <typename R> struct AdjArgs {
 
 // lin(x) = J_C(f(x))^T lam^{t+1}(x) from lam[19] = lam^{t+1}(x) (overwritten), stored to a.lin;
 // g gets the gradient terms of the links that x pulls through (x as the pulling site:
-// d f_q(x) / d s(x) on every link, plus the objective's force term)
-template <typename R>
-__device__ __forceinline__ void adj_collide_site(const AdjArgs<R> &a, const Nbr &nb, int i, int j, int k, int64_t x,
-                                                 R *lam, double &g)
+// d f_q(x) / d s(x) on every link, plus the objective's force term).  Of f only the moments are
+// kept; the source values and the site's own populations wait in registers for the gradient.
+template <bool BIG, bool ZERO, typename R>
+__device__ __forceinline__ void adj_collide_site(const AdjArgs<R> &a, const Site &p, R *lam, double &g)
 {
-    const int64_t st = a.g.stride;
-    // FP32 keeps each link's source value, source fraction and kind from the pull for the
-    // gradient terms; FP64 reads them again (cache hits) instead, which lowers its registers from
-    // 306 to 248 per lane (one to two wavefronts per SIMD).  Measured on MI355X (128 x 64 x 64):
-    // FP64 117.5 -> 112.6 us, while the FP32 kernel would go from 42 to 51-62 us.
     const double w = a.wobj;
-    if constexpr (sizeof(R) == 4) {
-        R f[19], sig[18], src[18], sy[18], out[19];
-        int kind[18];
-        grey_pull_links<R>(a.g, nb, i, j, k, x, f, sig, src, sy, kind);
-        collide_adj<R>(f, lam, a.g.omega, out);
+    R src[18], own[18], sy[18];
+    sources<BIG>(a.g, p, src);
 #pragma unroll
-        for (int q = 0; q < 19; ++q) a.lin[q * st + x] = out[q];
+    for (int q = 0; q < 18; ++q) own[q] = ldg<BIG>(a.g.A + kOPP[q] * a.g.stride, p.x);
+    R rho = 0, jx = 0, jy = 0, jz = 0;
+    R sx = R(0);
+    if constexpr (!ZERO) sx = ldg<BIG>(a.g.s, p.x);
 #pragma unroll
-        for (int q = 0; q < 18; ++q) {
-            const double L = (double)out[q];
-            const double abar = (double)a.g.a(kOPP[q], x);
-            const double syq = (double)sy[q];
-            g += L * (abar - (double)src[q]) * (1.0 - syq);
-            if (kind[q] == 0 && w != 0.0) g += w * kCX[q] * ((double)src[q] - abar) * (1.0 - syq);
+    for (int q = 0; q < 18; ++q) {
+        R f = src[q];
+        sy[q] = R(0);
+        if constexpr (!ZERO) {
+            sy[q] = source_s<BIG>(a.g, p, q);
+            const R sg = R(1) - (R(1) - sx) * (R(1) - sy[q]);
+            f = (R(1) - sg) * f + sg * own[q];
         }
-    } else {
-        R f[19];
-        grey_pull<R>(a.g, nb, i, j, k, x, f);
-        collide_adj<R>(f, lam, a.g.omega, lam); // in place: out[p] reads only lam[p] after the sums
+        rho += f;
+        if (kCX[q]) jx = kCX[q] > 0 ? jx + f : jx - f;
+        if (kCY[q]) jy = kCY[q] > 0 ? jy + f : jy - f;
+        if (kCZ[q]) jz = kCZ[q] > 0 ? jz + f : jz - f;
+    }
+    rho += ldg<BIG>(a.g.A + 18 * a.g.stride, p.x);
+    collide_adj<R>(rho, jx, jy, jz, a.g.omega, lam);
+    if (p.valid) {
 #pragma unroll
-        for (int q = 0; q < 19; ++q) a.lin[q * st + x] = lam[q];
+        for (int q = 0; q < 19; ++q) stg<BIG>(a.lin + q * a.g.stride, p.x, lam[q]);
+    }
 #pragma unroll
-        for (int q = 0; q < 18; ++q) {
-            R sv, syv;
-            int kd;
-            grey_link<R>(a.g, nb, i, j, k, q, sv, syv, kd);
-            const double L = (double)lam[q];
-            const double abar = (double)a.g.a(kOPP[q], x);
-            const double syq = (double)syv;
-            g += L * (abar - (double)sv) * (1.0 - syq);
-            if (kd == 0 && w != 0.0) g += w * kCX[q] * ((double)sv - abar) * (1.0 - syq);
-        }
+    for (int q = 0; q < 18; ++q) {
+        // (L - w c_x) (abar - src) (1 - s(y)); the objective's term on interior links only
+        double L = (double)lam[q];
+        if (kCX[q] && w != 0.0 && !p.ghost(-kCX[q])) L -= w * kCX[q];
+        double d = L * ((double)own[q] - (double)src[q]);
+        if constexpr (!ZERO) d *= 1.0 - (double)sy[q];
+        g += d;
     }
 }
 
 // lam^t(z) into lam[19]: the transposed pull gathered from a.lin at the sites z + c_p that pull
 // from z, the outlet-equilibrium transpose on the last x column and the objective's force term;
 // g gets the gradient terms of the links of which z is the source
-template <typename R>
-__device__ __forceinline__ void adj_stream_site(const AdjArgs<R> &a, const Nbr &nb, int i, int j, int k, int64_t z,
-                                                R *lam, double &g)
+template <bool BIG, bool ZERO, typename R>
+__device__ __forceinline__ void adj_stream_site(const AdjArgs<R> &a, const Site &z, R *lam, double &g)
 {
-    const int l = a.g.l;
     const int64_t st = a.g.stride;
     const double w = a.wobj;
-    const R sz = a.g.s[z];
+    R sz = R(0);
+    if constexpr (!ZERO) sz = ldg<BIG>(a.g.s, z.x);
 #pragma unroll
     for (int p = 0; p < 18; ++p) {
         const int pb = kOPP[p];
-        const int64_t zp = nb.at(i, j, k, kCX[p], kCY[p], kCZ[p]); // the site pulling p from z
-        double lp;
-        if (zp >= 0) {
-            const R s2 = a.g.s[zp];
-            const double sl = 1.0 - (1.0 - (double)sz) * (1.0 - (double)s2);
-            const double Lp = (double)a.lin[p * st + zp];
-            lp = (1.0 - sl) * Lp + sl * (double)a.lin[pb * st + z];
-            if (w != 0.0) lp += 2.0 * w * sl * kCX[p];
-            const double d = (double)a.g.a(pb, zp) - (double)a.g.a(p, z);
-            g += Lp * d * (1.0 - (double)s2);
-            if (w != 0.0) g -= w * kCX[p] * d * (1.0 - (double)s2);
+        const uint32_t zp = z.at(kCX[p], kCY[p], kCZ[p]); // the site pulling p from z
+        const bool gh = z.ghost(kCX[p]);
+        const double Lp = (double)ldg<BIG>(a.lin + p * st, zp);
+        const double d = (double)ldg<BIG>(a.g.A + pb * st, zp) - (double)ldg<BIG>(a.g.A + p * st, z.x);
+        double lp = Lp, e = Lp;
+        if (kCX[p] && w != 0.0) e -= w * kCX[p];
+        e *= d;
+        if constexpr (!ZERO) {
+            const double s2 = (double)ldg<BIG>(a.g.s, zp), own = (double)ldg<BIG>(a.lin + pb * st, z.x);
+            const double sl = 1.0 - (1.0 - (double)sz) * (1.0 - s2);
+            lp = (1.0 - sl) * Lp + sl * own;
+            if (kCX[p] && w != 0.0) lp += 2.0 * w * sl * kCX[p];
+            lp = gh ? (double)sz * own : lp; // ghost link: sigma = s(z)
+            e *= 1.0 - s2;
         } else {
-            lp = (double)sz * (double)a.lin[pb * st + z]; // ghost link: sigma = s(z)
+            lp = gh ? 0.0 : lp;
         }
+        g += gh ? 0.0 : e;
         lam[p] = (R)lp;
     }
-    lam[18] = a.lin[18 * st + z];
-    // outlet equilibrium transpose: z on the last x column feeds the ghost values read by the
-    // sites x = (l-1, j + cy, k + cz) for q = 10..14 (0-based 9..13)
-    if (a.g.xopen && i == l - 1) {
-        double Jx = 0, Jy = 0, Jz = 0;
+    lam[18] = ldg<BIG>(a.lin + 18 * st, z.x);
+    // Outlet equilibrium transpose: z on the last x column feeds the ghost values read by the sites
+    // x = (l-1, j + cy, k + cz) for q = 10..14 (0-based 9..13).  With Lw_q = w_q (1 - s(x)) lin_q(x):
+    //   lam_p += sum_q Lw_q (3 c_q.c_p + 9 (c_q.J) (c_q.c_p) - 3 J.c_p) = c_p . V
+    if (z.last) {
+        double J[3] = {0.0, 0.0, 0.0};
 #pragma unroll
-        for (int p = 0; p < 19; ++p) {
-            const double yp = (double)a.g.a(p, z);
-            Jx += kCX[p] * yp;
-            Jy += kCY[p] * yp;
-            Jz += kCZ[p] * yp;
+        for (int p = 0; p < 18; ++p) {
+            const double yp = (double)ldg<BIG>(a.g.A + p * st, z.x);
+            if (kCX[p]) J[0] += kCX[p] * yp;
+            if (kCY[p]) J[1] += kCY[p] * yp;
+            if (kCZ[p]) J[2] += kCZ[p] * yp;
         }
-        double Lw[5], cJ[5];
+        double V[3] = {0.0, 0.0, 0.0}, sum = 0.0;
 #pragma unroll
         for (int q = 9; q < 14; ++q) {
-            const int64_t x = nb.at(l - 1, j, k, 0, kCY[q], kCZ[q]);
-            const double sg = (double)a.g.s[x]; // sigma of the ghost link
-            const double L = (1.0 - sg) * (double)a.lin[q * st + x];
-            Lw[q - 9] = L * (double)wq<double>(q);
-            cJ[q - 9] = kCX[q] * Jx + kCY[q] * Jy + kCZ[q] * Jz;
+            const uint32_t x = z.at(0, kCY[q], kCZ[q]);
+            const double sg = (double)ldg<BIG>(a.g.s, x); // sigma of the ghost link
+            const double Lw = (1.0 - sg) * (double)ldg<BIG>(a.lin + q * st, x) * wq<double>(q);
+            const double t = Lw * (3.0 + 9.0 * (kCX[q] * J[0] + kCY[q] * J[1] + kCZ[q] * J[2]));
+            sum += Lw;
+            if (kCX[q]) V[0] += kCX[q] * t;
+            if (kCY[q]) V[1] += kCY[q] * t;
+            if (kCZ[q]) V[2] += kCZ[q] * t;
         }
-        // per population p the five terms in the order q = 10..14, one p at a time
+        for (int c = 0; c < 3; ++c) V[c] -= 3.0 * sum * J[c];
 #pragma unroll
-        for (int p = 0; p < 19; ++p) {
-            const double Jc = Jx * kCX[p] + Jy * kCY[p] + Jz * kCZ[p];
-            double acc = 0.0;
-#pragma unroll
-            for (int q = 9; q < 14; ++q) {
-                const double cc = kCX[q] * kCX[p] + kCY[q] * kCY[p] + kCZ[q] * kCZ[p];
-                acc += Lw[q - 9] * (3.0 * cc + 9.0 * cJ[q - 9] * cc - 3.0 * Jc);
-            }
-            lam[p] = (R)((double)lam[p] + acc);
-        }
+        for (int p = 0; p < 18; ++p)
+            lam[p] = (R)((double)lam[p] + (kCX[p] * V[0] + kCY[p] * V[1] + kCZ[p] * V[2]));
     }
-}
-
-// one thread per site: (i, j, k) of site x, false past the lattice
-__device__ __forceinline__ bool site_of(int l, int m, int n, int64_t &x, int &i, int &j, int &k)
-{
-    x = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (x >= (int64_t)l * m * n) return false;
-    i = (int)(x % l);
-    const int64_t r = x / l;
-    j = (int)(r % m);
-    k = (int)(r / m);
-    return true;
 }
 
 // the collide half of an adjoint step on its own: lin = J_C^T lam_in, and the gradient terms of
-// the links that x pulls through.  The same arithmetic as adj_collide_site written out with lam
-// read after the pull: built on adj_collide_site the FP32 kernel takes 170 registers per lane
-// instead of 166 (two wavefronts per SIMD instead of three; 47 against 42 us on 128 x 64 x 64).
-template <typename R> __global__ __launch_bounds__(256) void k_adj_collide(AdjArgs<R> a)
+// the links that x pulls through
+template <typename R, bool BIG> __global__ __launch_bounds__(256) void k_adj_collide(AdjArgs<R> a)
 {
-    const int64_t x = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t N = (int64_t)a.g.l * a.g.m * a.g.n;
-    if (x >= N) return;
-    const int i = (int)(x % a.g.l);
-    const int64_t r = x / a.g.l;
-    const int j = (int)(r % a.g.m), k = (int)(r / a.g.m);
-    const int64_t st = a.g.stride;
-    Nbr nb{a.g.l, a.g.m, a.g.n, a.g.xopen};
-    const double w = a.wobj;
+    const Site p = site_of(a.g);
+    R lam[19];
+#pragma unroll
+    for (int q = 0; q < 19; ++q) lam[q] = ldg<BIG>(a.lam_in + q * a.g.stride, p.x);
     double g = 0.0;
-    if constexpr (sizeof(R) == 4) {
-        R f[19], sig[18], src[18], sy[18], lam[19], out[19];
-        int kind[18];
-        grey_pull_links<R>(a.g, nb, i, j, k, x, f, sig, src, sy, kind);
-#pragma unroll
-        for (int q = 0; q < 19; ++q) lam[q] = a.lam_in[q * st + x];
-        collide_adj<R>(f, lam, a.g.omega, out);
-#pragma unroll
-        for (int q = 0; q < 19; ++q) a.lin[q * st + x] = out[q];
-#pragma unroll
-        for (int q = 0; q < 18; ++q) {
-            const double L = (double)out[q];
-            const double abar = (double)a.g.a(kOPP[q], x);
-            const double syq = (double)sy[q];
-            g += L * (abar - (double)src[q]) * (1.0 - syq);
-            if (kind[q] == 0 && w != 0.0) g += w * kCX[q] * ((double)src[q] - abar) * (1.0 - syq);
-        }
-    } else {
-        R f[19], lam[19];
-        grey_pull<R>(a.g, nb, i, j, k, x, f);
-#pragma unroll
-        for (int q = 0; q < 19; ++q) lam[q] = a.lam_in[q * st + x];
-        collide_adj<R>(f, lam, a.g.omega, lam); // in place: out[p] reads only lam[p] after the sums
-#pragma unroll
-        for (int q = 0; q < 19; ++q) a.lin[q * st + x] = lam[q];
-#pragma unroll
-        for (int q = 0; q < 18; ++q) {
-            R sv, syv;
-            int kd;
-            grey_link<R>(a.g, nb, i, j, k, q, sv, syv, kd);
-            const double L = (double)lam[q];
-            const double abar = (double)a.g.a(kOPP[q], x);
-            const double syq = (double)syv;
-            g += L * (abar - (double)sv) * (1.0 - syq);
-            if (kd == 0 && w != 0.0) g += w * kCX[q] * ((double)sv - abar) * (1.0 - syq);
-        }
-    }
-    a.gs[x] += g;
+    if (chunk_zero(a.g, p)) adj_collide_site<BIG, true>(a, p, lam, g);
+    else adj_collide_site<BIG, false>(a, p, lam, g);
+    if (p.valid) a.gs[p.x] += g;
 }
 
 // the stream half of an adjoint step on its own: lam_out = P^T lin (+ objective terms)
-template <typename R> __global__ __launch_bounds__(256) void k_adj_stream(AdjArgs<R> a)
+template <typename R, bool BIG> __global__ __launch_bounds__(256) void k_adj_stream(AdjArgs<R> a)
 {
-    int64_t z;
-    int i, j, k;
-    if (!site_of(a.g.l, a.g.m, a.g.n, z, i, j, k)) return;
-    const int64_t st = a.g.stride;
-    Nbr nb{a.g.l, a.g.m, a.g.n, a.g.xopen};
+    const Site z = site_of(a.g);
     R lam[19];
     double g = 0.0;
-    adj_stream_site<R>(a, nb, i, j, k, z, lam, g);
+    if (chunk_zero(a.g, z)) adj_stream_site<BIG, true>(a, z, lam, g);
+    else adj_stream_site<BIG, false>(a, z, lam, g);
+    if (!z.valid) return;
 #pragma unroll
-    for (int p = 0; p < 19; ++p) a.lam_out[p * st + z] = lam[p];
-    a.gs[z] += g;
+    for (int p = 0; p < 19; ++p) stg<BIG>(a.lam_out + p * a.g.stride, z.x, lam[p]);
+    a.gs[z.x] += g;
 }
 
 // the stream half of step t (sa: state a^t, lin^t in sa.lin) and the collide half of step t - 1
 // (ca: state a^{t-1}, lin^{t-1} into ca.lin) in one pass: lam^t stays in registers, so the
 // adjoint field is read and written once per step instead of twice.  The gradient sum of each
 // site takes the two halves' terms in the same order as the split kernels, so the result is
-// bit-identical to running k_adj_stream(t) and k_adj_collide(t - 1).
-template <typename R> __global__ __launch_bounds__(256) void k_adj_fused(AdjArgs<R> sa, AdjArgs<R> ca)
+// bit-identical to running k_adj_stream(t) and k_adj_collide(t - 1).  Bound by latency at two (FP32, 251
+// registers) and one (FP64) wavefronts per SIMD with every load of a half in flight: held to three
+// wavefronts, or with the loads in groups of 6, it spills or waits more (FP32 45 us; 65-90 us at
+// three).
+template <typename R, bool BIG> __global__ __launch_bounds__(256) void k_adj_fused(AdjArgs<R> sa, AdjArgs<R> ca)
 {
-    int64_t z;
-    int i, j, k;
-    if (!site_of(sa.g.l, sa.g.m, sa.g.n, z, i, j, k)) return;
-    Nbr nb{sa.g.l, sa.g.m, sa.g.n, sa.g.xopen};
+    const Site z = site_of(sa.g);
     R lam[19];
     double g1 = 0.0, g2 = 0.0;
-    adj_stream_site<R>(sa, nb, i, j, k, z, lam, g1);
-    adj_collide_site<R>(ca, nb, i, j, k, z, lam, g2);
-    double v = sa.gs[z];
+    if (chunk_zero(sa.g, z)) {
+        adj_stream_site<BIG, true>(sa, z, lam, g1);
+        adj_collide_site<BIG, true>(ca, z, lam, g2);
+    } else {
+        adj_stream_site<BIG, false>(sa, z, lam, g1);
+        adj_collide_site<BIG, false>(ca, z, lam, g2);
+    }
+    if (!z.valid) return;
+    double v = sa.gs[z.x];
     v += g1;
     v += g2;
-    sa.gs[z] = v;
+    sa.gs[z.x] = v;
 }
 
 // objective seed at t1: lam = w dF/da, gs += w dF/ds
-template <typename R> __global__ __launch_bounds__(256) void k_force_adj_seed(AdjArgs<R> a)
+template <typename R, bool BIG> __global__ __launch_bounds__(256) void k_force_adj_seed(AdjArgs<R> a)
 {
-    const int64_t z = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int l = a.g.l, m = a.g.m, n = a.g.n;
-    const int64_t N = (int64_t)l * m * n;
-    if (z >= N) return;
-    const int i = (int)(z % l);
-    const int64_t r = z / l;
-    const int j = (int)(r % m), k = (int)(r / m);
+    const Site z = site_of(a.g);
+    if (!z.valid) return;
     const int64_t st = a.g.stride;
-    Nbr nb{l, m, n, a.g.xopen};
     const double w = a.wobj;
-    const double sz = (double)a.g.s[z];
+    const double sz = (double)ldg<BIG>(a.g.s, z.x);
     double g = 0.0;
 #pragma unroll
     for (int q = 0; q < 18; ++q) { // z as x: pair (z, q) with interior source y = z - c_q
-        const int64_t y = nb.at(i, j, k, -kCX[q], -kCY[q], -kCZ[q]);
-        if (y < 0) continue;
-        const double d = (double)a.g.a(q, y) - (double)a.g.a(kOPP[q], z);
-        g += w * kCX[q] * d * (1.0 - (double)a.g.s[y]);
+        if (!kCX[q] || z.ghost(-kCX[q])) continue;
+        const uint32_t y = z.at(-kCX[q], -kCY[q], -kCZ[q]);
+        const double d = (double)ldg<BIG>(a.g.A + q * st, y) - (double)ldg<BIG>(a.g.A + kOPP[q] * st, z.x);
+        g += w * kCX[q] * d * (1.0 - (double)ldg<BIG>(a.g.s, y));
     }
 #pragma unroll
     for (int p = 0; p < 18; ++p) {
-        const int64_t zp = nb.at(i, j, k, kCX[p], kCY[p], kCZ[p]);
         double lam = 0.0;
-        if (zp >= 0) {
-            const double s2 = (double)a.g.s[zp];
+        if (kCX[p] && !z.ghost(kCX[p])) {
+            const uint32_t zp = z.at(kCX[p], kCY[p], kCZ[p]);
+            const double s2 = (double)ldg<BIG>(a.g.s, zp);
             const double sl = 1.0 - (1.0 - sz) * (1.0 - s2);
             lam = 2.0 * w * sl * kCX[p];
-            const double d = (double)a.g.a(p, z) - (double)a.g.a(kOPP[p], zp);
+            const double d = (double)ldg<BIG>(a.g.A + p * st, z.x) - (double)ldg<BIG>(a.g.A + kOPP[p] * st, zp);
             g += w * kCX[p] * d * (1.0 - s2);
         }
-        a.lam_out[p * st + z] = (R)lam;
+        stg<BIG>(a.lam_out + p * st, z.x, (R)lam);
     }
-    a.lam_out[18 * st + z] = R(0);
-    a.gs[z] += g;
+    stg<BIG>(a.lam_out + 18 * st, z.x, R(0));
+    a.gs[z.x] += g;
 }
+
+// the chunks of 64 sites without solid fraction in or next to them
+template <typename R> __global__ __launch_bounds__(256) void k_grey_chunks(GArgs<R> a, uint8_t *zero)
+{
+    const Site p = site_of(a);
+    bool any = a.s[p.x] != R(0);
+#pragma unroll
+    for (int q = 0; q < 18; ++q) any = any || a.s[p.at(kCX[q], kCY[q], kCZ[q])] != R(0);
+    const uint64_t b = __ballot(any);
+    if (p.valid && (threadIdx.x & 63) == 0) zero[p.x >> 6] = b == 0;
+}
+
+__global__ void k_to_f32(const double *src, float *dst, int64_t N)
+{
+    const int64_t x = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (x < N) dst[x] = (float)src[x];
+}
+
+__global__ void k_fill0(double *p, int64_t N)
+{
+    const int64_t x = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (x < N) p[x] = 0.0;
+}
+
+unsigned blocks_of(int64_t n) { return (unsigned)((n + 255) / 256); }
 
 template <typename R> GArgs<R> gargs(Handle *h, const void *from, void *to)
 {
@@ -544,6 +539,8 @@ template <typename R> GArgs<R> gargs(Handle *h, const void *from, void *to)
     a.B = static_cast<R *>(to);
     a.stride = h->stride;
     a.s = static_cast<const R *>(h->grey);
+    a.zero = h->grey_zero;
+    a.partial = h->diag;
     R inl[5];
     inlet_eq<R>((R)h->cfg.u_inflow, inl);
     for (int u = 0; u < 5; ++u) a.inl[u] = inl[u];
@@ -552,214 +549,212 @@ template <typename R> GArgs<R> gargs(Handle *h, const void *from, void *to)
     a.m = h->g.m;
     a.n = h->g.n;
     a.xopen = h->cfg.front != EUP_FACE_PERIODIC;
+    a.dl = UDiv::make((uint32_t)a.l);
+    a.dm = UDiv::make((uint32_t)a.m);
     return a;
 }
 
-template <typename R> unsigned grid_sites(Handle *h) { return (unsigned)((h->g.sites + 255) / 256); }
+// f(std::bool_constant<BIG>): arrays of 4 GiB and more take 64-bit offsets
+template <typename R, typename F> void by_size(Handle *h, F &&f)
+{
+    if ((uint64_t)h->g.sites * sizeof(R) < (1ull << 32)) f(std::false_type{});
+    else f(std::true_type{});
+}
 
-constexpr int kForceBlocks = 1024;
+// one step (to != null), the first nf force components of `from` added to the blocks' partial sums,
+// or both (the objective needs F_x alone)
+template <typename R> void launch_grey(Handle *h, const void *from, void *to, int nf)
+{
+    const GArgs<R> a = gargs<R>(h, from, to);
+    const dim3 grid(blocks_of(h->g.sites)), block(256);
+    by_size<R>(h, [&](auto big) {
+        constexpr bool B = decltype(big)::value;
+        if (to && nf) hipLaunchKernelGGL((k_grey<R, B, true, 1>), grid, block, 0, h->stream, a);
+        else if (to) hipLaunchKernelGGL((k_grey<R, B, true, 0>), grid, block, 0, h->stream, a);
+        else if (nf == 1) hipLaunchKernelGGL((k_grey<R, B, false, 1>), grid, block, 0, h->stream, a);
+        else hipLaunchKernelGGL((k_grey<R, B, false, 3>), grid, block, 0, h->stream, a);
+    });
+}
+
+// the outlet plane of the handle's current state, after the host set populations
+template <typename R> void refresh_outlet(Handle *h)
+{
+    if (h->outlet_dirty && h->cfg.front != EUP_FACE_PERIODIC)
+        hipLaunchKernelGGL((k_grey_outlet<R>), dim3(blocks_of((int64_t)h->g.m * h->g.n)), dim3(256), 0, h->stream,
+                           static_cast<R *>(h->buf[h->cur]), h->stride, h->g.l, h->g.m, h->g.n);
+    h->outlet_dirty = false;
+}
 
 template <typename R> int grey_step_t(Handle *h)
 {
-    GArgs<R> a = gargs<R>(h, h->buf[h->cur], h->buf[h->cur ^ 1]);
-    hipLaunchKernelGGL((k_grey_step<R>), dim3(grid_sites<R>(h)), dim3(256), 0, h->stream, a);
+    refresh_outlet<R>(h);
+    launch_grey<R>(h, h->buf[h->cur], h->buf[h->cur ^ 1], 0);
     if (hip_check(h, hipGetLastError(), "grey step")) return EUP_EHIP;
     h->cur ^= 1;
     return 0;
 }
 
-template <typename R> int force_into(Handle *h, const void *state, double weight, double *acc, double *last)
+// the blocks' partial force sums, cleared, and three results after them
+int force_scratch(Handle *h, double **sum)
 {
-    GArgs<R> a = gargs<R>(h, state, nullptr);
-    hipLaunchKernelGGL((k_grey_force<R>), dim3(kForceBlocks), dim3(256), 0, h->stream, a, h->diag);
-    hipLaunchKernelGGL(k_force_acc, dim3(1), dim3(256), 0, h->stream, h->diag, kForceBlocks, weight, acc, last);
-    return hip_check(h, hipGetLastError(), "grey force") ? EUP_EHIP : 0;
+    const int64_t np = 3 * (int64_t)blocks_of(h->g.sites), len = np + 3;
+    if (h->diag_len < len) {
+        hipFree(h->diag);
+        h->diag = nullptr;
+        h->diag_len = 0;
+        if (hip_check(h, hipMalloc((void **)&h->diag, sizeof(double) * len), "hipMalloc")) return EUP_EHIP;
+        h->diag_len = len;
+    }
+    hipLaunchKernelGGL(k_fill0, dim3(blocks_of(np)), dim3(256), 0, h->stream, h->diag, np);
+    *sum = h->diag + np;
+    return hip_check(h, hipGetLastError(), "force scratch") ? EUP_EHIP : 0;
 }
+
+int force_result(Handle *h, double *sum, double F[3])
+{
+    hipLaunchKernelGGL(k_force_sum, dim3(1), dim3(1024), 0, h->stream, h->diag, (int)blocks_of(h->g.sites), sum);
+    if (hip_check(h, hipGetLastError(), "grey force") ||
+        hip_check(h, hipMemcpyAsync(F, sum, sizeof(double) * 3, hipMemcpyDeviceToHost, h->stream), "copy") ||
+        hip_check(h, hipStreamSynchronize(h->stream), "sync"))
+        return EUP_EHIP;
+    return 0;
+}
+
+template <typename R> int grey_force_t(Handle *h, double F[3])
+{
+    double *sum;
+    if (int rc = force_scratch(h, &sum)) return rc;
+    refresh_outlet<R>(h);
+    launch_grey<R>(h, h->buf[h->cur], nullptr, 3);
+    return force_result(h, sum, F);
+}
+
+// A handle keeps its objective's device memory for the next call if it is at most this much
+// (allocating and freeing on each call: 128 x 64 x 64 FP32, 100 steps, 8.60 against 8.03 ms).
+constexpr size_t kKeepBytes = size_t(2) << 30;
 
 template <typename R>
 int objective_t(Handle *h, int t0, int t1, int K, double norm, double *J, void *grad_dev, int gdtype,
                 double *grad_host)
 {
     const int64_t N = h->g.sites;
-    const size_t S = sizeof(R) * (size_t)h->stride * 19; // one state
-    const int nck = t1 / K + 1;
+    const size_t S = (grey_state_bytes(h) + 255) / 256 * 256; // one state with its outlet plane
     const bool want_grad = grad_dev || grad_host;
-    std::vector<void *> mem;
-    auto alloc = [&](size_t bytes) -> void * {
-        void *p = nullptr;
-        if (hipMalloc(&p, bytes) != hipSuccess) return nullptr;
-        mem.push_back(p);
+    double *sum;
+    if (int rc = force_scratch(h, &sum)) return rc;
+    // Checkpoints: the states K, 2 K, ... up to t1 - 1, written by the forward sweep in place (state 0
+    // is the handle's own).  A segment's other states, at most min(K, t1) - 1; the forward sweep leaves
+    // those of the last segment there.  Two states for the rest of the forward sweep, the last one t1.
+    const int ncheck = want_grad ? (t1 - 1) / K : 0, nseg = want_grad ? (K < t1 ? K : t1) - 1 : 0;
+    const size_t gbytes = want_grad ? (sizeof(double) * (size_t)N + 255) / 256 * 256 : 0;
+    const size_t need = S * (size_t)(ncheck + nseg + 2 + (want_grad ? 3 : 0)) + gbytes;
+    if (h->work_len < need) {
+        hipFree(h->work);
+        h->work = nullptr;
+        h->work_len = 0;
+        if (hipMalloc(&h->work, need) != hipSuccess) {
+            (void)hipGetLastError();
+            h->work = nullptr;
+            return fail(h, EUP_EHIP, "eup_grey_objective: out of device memory for checkpoints and the adjoint");
+        }
+        h->work_len = need;
+    }
+    struct Give { // back after the call, unless small
+        Handle *h;
+        ~Give()
+        {
+            if (h->work_len <= kKeepBytes) return;
+            hipStreamSynchronize(h->stream);
+            hipFree(h->work);
+            h->work = nullptr;
+            h->work_len = 0;
+        }
+    } give{h};
+    char *mem = static_cast<char *>(h->work);
+    auto take = [&](size_t states) {
+        char *p = mem;
+        mem += S * states;
         return p;
     };
-    auto cleanup = [&]() {
-        for (void *p : mem) hipFree(p);
+    char *const ck = take((size_t)ncheck), *const seg = take((size_t)nseg);
+    void *const work[2] = {take(1), take(1)};
+    refresh_outlet<R>(h);
+    const int tlast = want_grad ? ncheck * K : t1; // first state of the last segment
+    auto check = [&](int c) -> void * { return c == 0 ? h->buf[h->cur] : ck + S * (size_t)(c - 1); };
+    auto segment = [&](int t, int tb) -> void * { return t == tb ? check(tb / K) : seg + S * (size_t)(t - tb - 1); };
+    // where the forward sweep keeps state t
+    auto state = [&](int t) -> void * {
+        if (t == 0) return check(0);
+        if (want_grad && t < t1 && t % K == 0) return check(t / K);
+        if (want_grad && t > tlast && t < t1) return segment(t, tlast);
+        return work[t & 1];
     };
-    if (h->diag_len < 3 * kForceBlocks + 16) {
-        hipFree(h->diag);
-        h->diag = nullptr;
-        h->diag_len = 0;
-        if (hip_check(h, hipMalloc((void **)&h->diag, sizeof(double) * (3 * kForceBlocks + 16)), "hipMalloc"))
-            return EUP_EHIP;
-        h->diag_len = 3 * kForceBlocks + 16;
-    }
-    double *acc = h->diag + 3 * kForceBlocks;     // [0..2] accumulator, [3..5] last force
-    char *ck = static_cast<char *>(alloc(S * nck));
-    void *work[2] = {alloc(S), alloc(S)};
-    if (!ck || !work[0] || !work[1]) {
-        cleanup();
-        return fail(h, EUP_EHIP, "eup_grey_objective: out of device memory for checkpoints");
-    }
-    if (hip_check(h, hipMemsetAsync(acc, 0, sizeof(double) * 6, h->stream), "memset")) {
-        cleanup();
-        return EUP_EHIP;
-    }
-    // forward sweep from the current state
-    void *init = h->buf[h->cur];
-    if (hip_check(h, hipMemcpyAsync(work[0], init, S, hipMemcpyDeviceToDevice, h->stream), "copy")) {
-        cleanup();
-        return EUP_EHIP;
-    }
-    int c = 0;
-    for (int t = 0; t <= t1; ++t) {
-        void *cur = work[c];
-        if (t % K == 0 && hip_check(h, hipMemcpyAsync(ck + S * (size_t)(t / K), cur, S, hipMemcpyDeviceToDevice,
-                                                      h->stream), "checkpoint copy")) {
-            cleanup();
-            return EUP_EHIP;
-        }
-        if (t >= t0 && force_into<R>(h, cur, 1.0, acc, acc + 3)) {
-            cleanup();
-            return EUP_EHIP;
-        }
-        if (t == t1) break;
-        GArgs<R> a = gargs<R>(h, cur, work[c ^ 1]);
-        hipLaunchKernelGGL((k_grey_step<R>), dim3(grid_sites<R>(h)), dim3(256), 0, h->stream, a);
-        c ^= 1;
-    }
-    double sum[3];
-    if (hip_check(h, hipGetLastError(), "forward sweep") ||
-        hip_check(h, hipMemcpyAsync(sum, acc, sizeof(double) * 3, hipMemcpyDeviceToHost, h->stream), "copy") ||
-        hip_check(h, hipStreamSynchronize(h->stream), "sync")) {
-        cleanup();
-        return EUP_EHIP;
-    }
+    for (int t = 0; t < t1; ++t) launch_grey<R>(h, state(t), state(t + 1), t >= t0 ? 1 : 0);
+    launch_grey<R>(h, state(t1), nullptr, 1);
+    double F[3];
+    if (int rc = force_result(h, sum, F)) return rc;
     const double wobj = 1.0 / ((double)(t1 - t0 + 1) * norm);
-    *J = sum[0] * wobj;
-    if (want_grad) {
-        // a segment holds at most min(K, t1) forward states (t - tb < te - tb <= min(K, t1))
-        char *seg = static_cast<char *>(alloc(S * (size_t)(K < t1 ? K : t1)));
-        void *lam = alloc(S);                    // lam^t between the halves of a step
-        void *linb[2] = {alloc(S), alloc(S)};    // lin^t, lin^{t-1}
-        double *gs = static_cast<double *>(alloc(sizeof(double) * N));
-        if (!seg || !lam || !linb[0] || !linb[1] || !gs) {
-            cleanup();
-            return fail(h, EUP_EHIP, "eup_grey_objective: out of device memory for the adjoint");
-        }
-        if (hip_check(h, hipMemsetAsync(gs, 0, sizeof(double) * N, h->stream), "memset gradient")) {
-            cleanup();
-            return EUP_EHIP;
-        }
-        auto adj = [&](const void *state, const void *lam_in, void *lin, void *lam_out, double w) {
-            AdjArgs<R> q;
-            q.g = gargs<R>(h, state, nullptr);
-            q.lam_in = static_cast<const R *>(lam_in);
-            q.lin = static_cast<R *>(lin);
-            q.lam_out = static_cast<R *>(lam_out);
-            q.gs = gs;
-            q.wobj = w;
-            return q;
-        };
-        // seed at t1: recompute a^{t1} from its checkpoint
-        {
-            const int cc = t1 / K;
-            if (hip_check(h, hipMemcpyAsync(work[0], ck + S * (size_t)cc, S, hipMemcpyDeviceToDevice, h->stream),
-                          "checkpoint restore")) {
-                cleanup();
-                return EUP_EHIP;
-            }
-            int w = 0;
-            for (int t = cc * K; t < t1; ++t) {
-                GArgs<R> a = gargs<R>(h, work[w], work[w ^ 1]);
-                hipLaunchKernelGGL((k_grey_step<R>), dim3(grid_sites<R>(h)), dim3(256), 0, h->stream, a);
-                w ^= 1;
-            }
-            AdjArgs<R> q = adj(work[w], nullptr, nullptr, lam, wobj);
-            hipLaunchKernelGGL((k_force_adj_seed<R>), dim3(grid_sites<R>(h)), dim3(256), 0, h->stream, q);
-        }
-        // Per segment: the collide half of its last step, then the stream half of step t fused
-        // with the collide half of step t - 1 (both states are in the recomputed segment), then
-        // the stream half of its first step.  Fused by default in FP64 (MI355X, 128 x 64 x 64:
-        // 154 us against 102 + 71 us split); FP32 runs the halves on their own by default (fused
-        // 97 us against 47 + 44 us: the fused kernel's 173 registers per lane allow two
-        // wavefronts per SIMD, the split collide's three).  EUP_ADJ_FUSED=0 / 1 forces either
-        // form; both give the same results bit for bit.
-        bool fuse = sizeof(R) == 8;
-        if (const char *e = getenv("EUP_ADJ_FUSED")) fuse = atoi(e) != 0;
-        const dim3 grid(grid_sites<R>(h));
-        for (int cc = (t1 - 1) / K; cc >= 0; --cc) {
+    *J = F[0] * wobj;
+    if (!want_grad) return 0;
+    void *const lam = take(1);                    // lam^t between the halves of a step
+    void *const linb[2] = {take(1), take(1)};     // lin^t, lin^{t-1}
+    double *const gs = reinterpret_cast<double *>(mem);
+    const dim3 grid(blocks_of(N)), block(256);
+    hipLaunchKernelGGL(k_fill0, grid, block, 0, h->stream, gs, N);
+    auto adj = [&](const void *st, const void *lam_in, void *lin, void *lam_out, double w) {
+        AdjArgs<R> q;
+        q.g = gargs<R>(h, st, nullptr);
+        q.lam_in = static_cast<const R *>(lam_in);
+        q.lin = static_cast<R *>(lin);
+        q.lam_out = static_cast<R *>(lam_out);
+        q.gs = gs;
+        q.wobj = w;
+        return q;
+    };
+    // Per segment: the collide half of its last step, then the stream half of step t fused with the
+    // collide half of step t - 1 (both states are in the segment), then the stream half of its first
+    // step.  Fused, 128 x 64 x 64 (MI355X): FP32 45 us against 30 + 28 us apart, FP64 70 x 45 x 36 24.6
+    // against 15.2 + 13.1 us.  EUP_ADJ_FUSED=0 / 1 forces the halves apart or together; both give the
+    // same results bit for bit.
+    bool fuse = true;
+    if (const char *e = getenv("EUP_ADJ_FUSED")) fuse = atoi(e) != 0;
+    by_size<R>(h, [&](auto big) {
+        constexpr bool B = decltype(big)::value;
+        hipLaunchKernelGGL((k_force_adj_seed<R, B>), grid, block, 0, h->stream, adj(state(t1), nullptr, nullptr, lam, wobj));
+        for (int cc = ncheck; cc >= 0; --cc) {
             const int tb = cc * K, te = (cc + 1) * K < t1 ? (cc + 1) * K : t1;
-            if (te <= tb) continue; // no step in this segment (t1 >= 1 keeps every segment non-empty)
-            if (hip_check(h, hipMemcpyAsync(seg, ck + S * (size_t)cc, S, hipMemcpyDeviceToDevice, h->stream),
-                          "checkpoint restore")) {
-                cleanup();
-                return EUP_EHIP;
-            }
-            for (int t = tb + 1; t < te; ++t) {
-                GArgs<R> a = gargs<R>(h, seg + S * (size_t)(t - 1 - tb), seg + S * (size_t)(t - tb));
-                hipLaunchKernelGGL((k_grey_step<R>), grid, dim3(256), 0, h->stream, a);
-            }
-            auto at = [&](int t) { return static_cast<const void *>(seg + S * (size_t)(t - tb)); };
+            if (cc < ncheck) // the last segment's states are those of the forward sweep
+                for (int t = tb + 1; t < te; ++t) launch_grey<R>(h, segment(t - 1, tb), segment(t, tb), 0);
+            auto at = [&](int t) { return static_cast<const void *>(segment(t, tb)); };
             auto wt = [&](int t) { return t >= t0 ? wobj : 0.0; };
             int b = 0; // linb[b] holds lin^t
-            hipLaunchKernelGGL((k_adj_collide<R>), grid, dim3(256), 0, h->stream,
+            hipLaunchKernelGGL((k_adj_collide<R, B>), grid, block, 0, h->stream,
                                adj(at(te - 1), lam, linb[b], nullptr, wt(te - 1)));
             for (int t = te - 1; t > tb; --t) {
                 if (fuse) {
-                    hipLaunchKernelGGL((k_adj_fused<R>), grid, dim3(256), 0, h->stream,
+                    hipLaunchKernelGGL((k_adj_fused<R, B>), grid, block, 0, h->stream,
                                        adj(at(t), nullptr, linb[b], nullptr, wt(t)),
                                        adj(at(t - 1), nullptr, linb[b ^ 1], nullptr, wt(t - 1)));
                     b ^= 1;
                 } else {
-                    hipLaunchKernelGGL((k_adj_stream<R>), grid, dim3(256), 0, h->stream,
+                    hipLaunchKernelGGL((k_adj_stream<R, B>), grid, block, 0, h->stream,
                                        adj(at(t), nullptr, linb[b], lam, wt(t)));
-                    hipLaunchKernelGGL((k_adj_collide<R>), grid, dim3(256), 0, h->stream,
+                    hipLaunchKernelGGL((k_adj_collide<R, B>), grid, block, 0, h->stream,
                                        adj(at(t - 1), lam, linb[b], nullptr, wt(t - 1)));
                 }
             }
-            hipLaunchKernelGGL((k_adj_stream<R>), grid, dim3(256), 0, h->stream,
+            hipLaunchKernelGGL((k_adj_stream<R, B>), grid, block, 0, h->stream,
                                adj(at(tb), nullptr, linb[b], lam, wt(tb)));
         }
-        if (hip_check(h, hipGetLastError(), "adjoint sweep")) {
-            cleanup();
-            return EUP_EHIP;
-        }
-        int rc = 0;
-        if (grad_host) {
-            if (hip_check(h, hipMemcpyAsync(grad_host, gs, sizeof(double) * N, hipMemcpyDeviceToHost, h->stream), "copy grad"))
-                rc = EUP_EHIP;
-        } else if (gdtype == EUP_STORE_F64) {
-            if (hip_check(h, hipMemcpyAsync(grad_dev, gs, sizeof(double) * N, hipMemcpyDeviceToDevice, h->stream), "copy grad"))
-                rc = EUP_EHIP;
-        } else {
-            rc = 0;
-            float *gd = static_cast<float *>(grad_dev);
-            std::vector<double> tmp(N);
-            if (hip_check(h, hipMemcpyAsync(tmp.data(), gs, sizeof(double) * N, hipMemcpyDeviceToHost, h->stream), "copy") ||
-                hip_check(h, hipStreamSynchronize(h->stream), "sync"))
-                rc = EUP_EHIP;
-            std::vector<float> tf(N);
-            for (int64_t x = 0; x < N; ++x) tf[x] = (float)tmp[x];
-            if (!rc && hip_check(h, hipMemcpy(gd, tf.data(), sizeof(float) * N, hipMemcpyHostToDevice), "copy"))
-                rc = EUP_EHIP;
-        }
-        if (!rc && hip_check(h, hipStreamSynchronize(h->stream), "sync")) rc = EUP_EHIP;
-        if (rc) {
-            cleanup();
-            return rc;
-        }
-    }
-    cleanup();
-    return 0;
+    });
+    if (grad_dev && gdtype == EUP_STORE_F32)
+        hipLaunchKernelGGL(k_to_f32, grid, block, 0, h->stream, gs, static_cast<float *>(grad_dev), N);
+    if (hip_check(h, hipGetLastError(), "adjoint sweep")) return EUP_EHIP;
+    if ((grad_host || gdtype == EUP_STORE_F64) &&
+        hip_check(h, hipMemcpyAsync(grad_host ? (void *)grad_host : grad_dev, gs, sizeof(double) * N,
+                                    grad_host ? hipMemcpyDeviceToHost : hipMemcpyDeviceToDevice, h->stream), "copy grad"))
+        return EUP_EHIP;
+    return hip_check(h, hipStreamSynchronize(h->stream), "sync") ? EUP_EHIP : 0;
 }
 
 template <typename F> int rdispatch(Handle *h, F &&f)
@@ -789,6 +784,7 @@ int grey_set_field(Handle *h, const void *s, int dtype, bool on_device)
     const int64_t N = h->g.sites;
     const size_t rb = h->cfg.storage == EUP_STORE_F64 ? 8 : 4;
     if (!h->grey && hip_check(h, hipMalloc(&h->grey, rb * N), "hipMalloc grey")) return EUP_EHIP;
+    if (!h->grey_zero && hip_check(h, hipMalloc((void **)&h->grey_zero, (N + 63) / 64), "hipMalloc grey")) return EUP_EHIP;
     const void *src = s;
     void *tmp = nullptr;
     if (!on_device) {
@@ -806,6 +802,14 @@ int grey_set_field(Handle *h, const void *s, int dtype, bool on_device)
                            dtype, static_cast<R *>(h->grey), N);
         return hip_check(h, hipGetLastError(), "grey field") ? EUP_EHIP : 0;
     });
+    if (!rc) {
+        rc = rdispatch(h, [&](auto *p) {
+            using R = std::remove_pointer_t<decltype(p)>;
+            hipLaunchKernelGGL((k_grey_chunks<R>), dim3(blocks_of(N)), dim3(256), 0, h->stream,
+                               gargs<R>(h, nullptr, nullptr), h->grey_zero);
+            return hip_check(h, hipGetLastError(), "grey chunks") ? EUP_EHIP : 0;
+        });
+    }
     if (!rc && hip_check(h, hipStreamSynchronize(h->stream), "sync")) rc = EUP_EHIP;
     hipFree(tmp);
     return rc;
@@ -813,24 +817,7 @@ int grey_set_field(Handle *h, const void *s, int dtype, bool on_device)
 
 int grey_force(Handle *h, double F[3])
 {
-    if (h->diag_len < 3 * kForceBlocks + 16) {
-        hipFree(h->diag);
-        h->diag = nullptr;
-        h->diag_len = 0;
-        if (hip_check(h, hipMalloc((void **)&h->diag, sizeof(double) * (3 * kForceBlocks + 16)), "hipMalloc"))
-            return EUP_EHIP;
-        h->diag_len = 3 * kForceBlocks + 16;
-    }
-    double *acc = h->diag + 3 * kForceBlocks;
-    if (hip_check(h, hipMemsetAsync(acc, 0, sizeof(double) * 6, h->stream), "memset")) return EUP_EHIP;
-    int rc = rdispatch(h, [&](auto *p) {
-        return force_into<std::remove_pointer_t<decltype(p)>>(h, h->buf[h->cur], 1.0, acc, acc + 3);
-    });
-    if (rc) return rc;
-    if (hip_check(h, hipMemcpyAsync(F, acc + 3, sizeof(double) * 3, hipMemcpyDeviceToHost, h->stream), "copy") ||
-        hip_check(h, hipStreamSynchronize(h->stream), "sync"))
-        return EUP_EHIP;
-    return 0;
+    return rdispatch(h, [&](auto *p) { return grey_force_t<std::remove_pointer_t<decltype(p)>>(h, F); });
 }
 
 int grey_objective(Handle *h, int t0, int t1, int K, double norm, double *J, void *grad_dev, int gdtype,

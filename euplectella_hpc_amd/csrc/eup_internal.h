@@ -59,8 +59,8 @@ struct Handle {
     int64_t tiles_fluid = 0, tiles_mixed = 0, tiles_solid = 0;
     int32_t *mixed_list = nullptr; // tile indices of mixed tiles
     void *outlet[2] = {nullptr, nullptr}; // outlet ghost plane, 5 x m x n (compute type)
-    bool outlet_dirty = true;      // the host wrote populations: physics mode recomputes its outlet
-                                   // plane, parity mode refills the constant inflow plane
+    bool outlet_dirty = true;      // the host wrote populations: physics and grey mode recompute the
+                                   // outlet plane, parity mode refills the constant inflow plane
     size_t fused_lds = (size_t)-1; // dynamic LDS per block of the fused kernel (occupancy cap)
     int fused_remap = -1;          // fused kernel block order: 0 dispatch, 1 XCD-contiguous, 2 XCD-owned rows
     size_t parity_lds = (size_t)-1; // the same for the parity stream-collide kernel
@@ -70,7 +70,10 @@ struct Handle {
     double *site19 = nullptr;     // one site's 19 populations in FP64
     // grey mode
     void *grey = nullptr;         // solid fraction (compute type), l*m*n
+    uint8_t *grey_zero = nullptr; // per 64 sites: no solid fraction there or next to them
     bool grey_set = false;
+    void *work = nullptr;         // objective scratch kept between calls
+    size_t work_len = 0;
     int64_t device_bytes = 0;
 };
 
@@ -93,6 +96,8 @@ int init_equilibrium(Handle *h, double ux, double uy, double uz, double noise, u
 int parity_get_pop(Handle *h, int q);
 
 // grey mode (eup_grey.hip)
+// bytes of a grey state: 19 populations and the outlet ghost plane
+inline size_t grey_state_bytes(const Handle *h) { return h->elem * (19 * (size_t)h->stride + 5 * (size_t)h->g.m * h->g.n); }
 int grey_step(Handle *h);
 int grey_set_field(Handle *h, const void *s, int dtype, bool on_device);
 int grey_force(Handle *h, double F[3]);
