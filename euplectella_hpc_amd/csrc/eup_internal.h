@@ -79,6 +79,7 @@ struct Handle {
 
 int fail(Handle *h, int code, const std::string &msg);
 size_t occupancy_lds_bytes(const Handle *h, int cap);
+bool stream_stores(const Handle *h, double bytes);
 int hip_check(Handle *h, hipError_t e, const char *what);
 
 // parity mode (eup_parity.hip)

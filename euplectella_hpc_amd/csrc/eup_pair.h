@@ -139,15 +139,15 @@ template <typename S, int Q> __device__ __forceinline__ S raw_load_at(Rsrc r, ui
     return rsrc_load<S>(r, off + (b & 4095), b & ~4095);
 }
 
-template <typename S, int Q> __device__ __forceinline__ void raw_store_at(Rsrc r, uint32_t off, S v)
+template <typename S, bool NT, int Q> __device__ __forceinline__ void raw_store_at(Rsrc r, uint32_t off, S v)
 {
     constexpr int b = Q * kTile * (int)sizeof(S), lo = b & 4095, hi = b & ~4095;
-    constexpr int kNt = 2; // non-temporal
+    constexpr int aux = NT ? 2 : 0; // non-temporal
     if constexpr (sizeof(S) == 4) {
-        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), r, (int)(off + lo), hi, kNt);
+        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), r, (int)(off + lo), hi, aux);
     } else {
         typedef uint32_t u2 __attribute__((ext_vector_type(2)));
-        __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2, v), r, (int)(off + lo), hi, kNt);
+        __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2, v), r, (int)(off + lo), hi, aux);
     }
 }
 
@@ -261,13 +261,13 @@ __device__ __forceinline__ void pair_bounce(QSeq<Qs...>, uint32_t lm, const P &o
     ((x[Qs] = ((lm >> Qs) & 1u) ? b[Qs] : x[Qs]), ...);
 }
 
-template <typename S, int... Qs>
+template <typename S, bool NT, int... Qs>
 __device__ __forceinline__ void pair_store(QSeq<Qs...>, Rsrc r, uint32_t off, const S *x)
 {
-    (raw_store_at<S, Qs>(r, off, x[Qs]), ...);
+    (raw_store_at<S, NT, Qs>(r, off, x[Qs]), ...);
 }
 
-template <typename S, bool XOPEN>
+template <typename S, bool XOPEN, bool NT>
 __global__ __launch_bounds__((pair_threads<S>())) void k_pair(XArgs<S> a, PairMap pm)
 {
     extern __shared__ __align__(16) char pair_lds[];
@@ -453,7 +453,7 @@ __global__ __launch_bounds__((pair_threads<S>())) void k_pair(XArgs<S> a, PairMa
         pair_collide<S>(x2, a);
         const int ko = max(kz - 1, 0); // kz - 1, 0 <= ko < n, where a lane stores
         const bool out = it >= 2 && inner && !(lm_prev & 0x80000000u);
-        pair_store<S>(Q19{}, plane_of(B, ko, pm.plane), out ? w.xo[1] : kOutside, x2);
+        pair_store<S, NT>(Q19{}, plane_of(B, ko, pm.plane), out ? w.xo[1] : kOutside, x2);
         if constexpr (XOPEN) {
             if (out && at1) {
                 S o[5];

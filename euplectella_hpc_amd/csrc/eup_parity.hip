@@ -222,7 +222,8 @@ struct SegMap {
     uint32_t order; // 0 dispatch, 1 XCD-contiguous ranges of segments, 2 XCD-owned rows
 };
 
-__global__ __launch_bounds__(256) void k_stream_collide(PArgs a, SegMap s)
+// NT: non-temporal stores (stream_stores)
+template <bool NT> __global__ __launch_bounds__(256) void k_stream_collide(PArgs a, SegMap s)
 {
     // block order as in the physics kernel: hardware block b runs on XCD b % 8; order 2 deals
     // each group of 8 * grp blocks out so that every XCD takes a whole row (the lines that
@@ -251,10 +252,12 @@ __global__ __launch_bounds__(256) void k_stream_collide(PArgs a, SegMap s)
     pull_all(Q18{}, a, row, lp, lpmp, i, x);
     x[18] = (a.A0 + (18 * a.stride + row))[(uint64_t)(uint32_t)i];
     collide<double>(x, x, a.omega, a.fgrad);
-    // non-temporal: the next reads of these values come a step later
 #pragma unroll
-    for (int q = 0; q < 19; ++q)
-        __builtin_nontemporal_store(x[q], &(a.B0 + ((int64_t)q * a.stride + row))[(uint64_t)(uint32_t)i]);
+    for (int q = 0; q < 19; ++q) {
+        double *p = &(a.B0 + ((int64_t)q * a.stride + row))[(uint64_t)(uint32_t)i];
+        if constexpr (NT) __builtin_nontemporal_store(x[q], p);
+        else *p = x[q];
+    }
     if (i == a.l) {
         // the next step's outflow ghost values of this row (bcond.bc.F90:127-164), from the values
         // just stored; the ghost fill uses them unless bounce-back changes this site first
@@ -402,7 +405,13 @@ int parity_step(Handle *h)
         if (const char *e = getenv("EUP_PARITY_BLOCKS_PER_CU")) cap = atoi(e);
         h->parity_lds = occupancy_lds_bytes(h, cap);
     }
-    hipLaunchKernelGGL(k_stream_collide, dim3(8u * sm.chunk), dim3(256), h->parity_lds, h->stream, a, sm);
+    // us per step, non-temporal against cached: 128 x 64 x 64 42.0 / 33.8, 160 x 80 x 64 58.0 / 55.1, and, within
+    // the L2 caches (where stream_stores draws a line that is not needed here), 64 x 32 x 32 14.3 / 13.2
+    const double bytes = 2.0 * 19 * sizeof(double) * (double)h->stride;
+    if (stream_stores(h, bytes < 50e6 ? 50e6 : bytes))
+        hipLaunchKernelGGL((k_stream_collide<true>), dim3(8u * sm.chunk), dim3(256), h->parity_lds, h->stream, a, sm);
+    else
+        hipLaunchKernelGGL((k_stream_collide<false>), dim3(8u * sm.chunk), dim3(256), h->parity_lds, h->stream, a, sm);
     if (hip_check(h, hipGetLastError(), "parity step launch")) return EUP_EHIP;
     h->cur ^= 1;
     return 0;

@@ -233,20 +233,14 @@ __device__ __forceinline__ void x_edges(const XArgs<S> &a, const Wave &w, uint32
     (void)cxs;
 }
 
-#ifndef EUP_NT_STORE
-#define EUP_NT_STORE 1
-#endif
-
-template <typename S> __device__ __forceinline__ void store_val(S *p, S v)
+// NT: non-temporal
+template <bool NT, typename S> __device__ __forceinline__ void store_val(S *p, S v)
 {
-#if EUP_NT_STORE
-    if constexpr (std::is_same_v<S, bf16_t> || std::is_same_v<S, e3m12_t>)
+    if constexpr (!NT) *p = v;
+    else if constexpr (std::is_same_v<S, bf16_t> || std::is_same_v<S, e3m12_t>)
         __builtin_nontemporal_store(v.bits, reinterpret_cast<uint16_t *>(p));
     else
         __builtin_nontemporal_store(v, p);
-#else
-    *p = v;
-#endif
 }
 
 // the stored value of population Q from the kernel's representation
@@ -258,19 +252,19 @@ __device__ __forceinline__ void conv(const XArgs<S> &a, const typename Store<S>:
 }
 
 // convert population Q, keep the stored value in sv and store it
-template <typename S, int Q>
+template <typename S, bool NT, int Q>
 __device__ __forceinline__ void put(const XArgs<S> &a, char *tb, uint32_t o0, const typename Store<S>::compute *x,
                                     S *sv)
 {
     conv<S, Q>(a, x, sv);
-    store_val<S>(reinterpret_cast<S *>(tb + (int64_t)Q * kTile * sizeof(S) + (uint64_t)o0), sv[Q]);
+    store_val<NT>(reinterpret_cast<S *>(tb + (int64_t)Q * kTile * sizeof(S) + (uint64_t)o0), sv[Q]);
 }
 
-template <typename S, int... Qs>
+template <typename S, bool NT, int... Qs>
 __device__ __forceinline__ void put_all(QSeq<Qs...>, const XArgs<S> &a, char *tb, uint32_t o0,
                                         const typename Store<S>::compute *x, S *sv)
 {
-    (put<S, Qs>(a, tb, o0, x, sv), ...);
+    (put<S, NT, Qs>(a, tb, o0, x, sv), ...);
 }
 
 // The x = l sites write the next step's outlet ghost values (bcond.bc.F90:127-164) from their
@@ -304,18 +298,18 @@ __device__ __forceinline__ void outlet_next(const XArgs<S> &a, const Wave &w, in
 
 // Store the lane's post-collision populations x of tile t, converted once: the outlet (the x = l
 // sites) takes the values as stored.
-template <typename S, bool XOPEN>
+template <typename S, bool XOPEN, bool NT>
 __device__ __forceinline__ void finish(const XArgs<S> &a, uint32_t t, const Wave &w, int j, int k,
                                        const typename Store<S>::compute *x)
 {
     S sv[19];
-    put_all<S>(Q19{}, a, reinterpret_cast<char *>(a.B) + (int64_t)t * ((int64_t)kTileElems * sizeof(S)), w.o0, x, sv);
+    put_all<S, NT>(Q19{}, a, reinterpret_cast<char *>(a.B) + (int64_t)t * ((int64_t)kTileElems * sizeof(S)), w.o0, x, sv);
     if constexpr (XOPEN) outlet_next<S>(a, w, j, k, sv);
 }
 
 // Update tile t (addressing w, row j, k), one site per lane.  MIXED applies the link mask lm of the
 // lane's site: bounce-back from solid sources, solid sites frozen.
-template <typename S, bool XOPEN, bool MIXED>
+template <typename S, bool XOPEN, bool NT, bool MIXED>
 __device__ __forceinline__ void update_tile(const XArgs<S> &a, uint32_t t, const Wave &w, int j, int k,
                                             uint32_t lm)
 {
@@ -333,7 +327,7 @@ __device__ __forceinline__ void update_tile(const XArgs<S> &a, uint32_t t, const
     if constexpr (kTopTest<S>) x[18] = Store<S>::nan_if_top(top, x[18]);
     if constexpr (kOnStored<S>) collide_dev<Store<S>::deviation>(x, a.bgk);
     else collide<R>(x, x, a.omega, a.fgrad);
-    finish<S, XOPEN>(a, t, w, j, k, x);
+    finish<S, XOPEN, NT>(a, t, w, j, k, x);
 }
 
 // Mixed tile with every load issued at once: the link masks, the 19 pulls from the fluid
@@ -373,7 +367,7 @@ __device__ __forceinline__ void choose_all(QSeq<Qs...>, const XArgs<S> &a, uint3
     (choose<S, Qs>(a, lm, own, x), ...);
 }
 
-template <typename S, bool XOPEN>
+template <typename S, bool XOPEN, bool NT>
 __device__ __forceinline__ void update_mixed_at_once(const XArgs<S> &a, uint32_t t, const Wave &w, int j, int k,
                                                      const uint32_t *lmp)
 {
@@ -391,13 +385,13 @@ __device__ __forceinline__ void update_mixed_at_once(const XArgs<S> &a, uint32_t
     if constexpr (kTopTest<S>) x[18] = Store<S>::nan_if_top(top, x[18]);
     if constexpr (kOnStored<S>) collide_dev<Store<S>::deviation>(x, a.bgk);
     else collide<R>(x, x, a.omega, a.fgrad);
-    finish<S, XOPEN>(a, t, w, j, k, x);
+    finish<S, XOPEN, NT>(a, t, w, j, k, x);
 }
 
 template <typename S> constexpr bool kMixedAtOnce = sizeof(S) <= 4;
 
 // One step of one tile per wavefront (the body of k_fused).
-template <typename S, bool XOPEN>
+template <typename S, bool XOPEN, bool NT>
 __device__ __forceinline__ void fused_step(const XArgs<S> &a)
 {
     // Block order (chosen by fused_block_order).  Hardware block b runs on XCD b % 8.  Order 0:
@@ -430,22 +424,22 @@ __device__ __forceinline__ void fused_step(const XArgs<S> &a)
     wave_setup<S>(a, w, ti, j, k, (int)(threadIdx.x & 63));
     if (code == kTileSolid) return;
     if (code == kTileFluid) {
-        update_tile<S, XOPEN, false>(a, t, w, j, k, 0u);
+        update_tile<S, XOPEN, NT, false>(a, t, w, j, k, 0u);
     } else if constexpr (kMixedAtOnce<S>) {
-        update_mixed_at_once<S, XOPEN>(a, t, w, j, k, a.link + ((size_t)code * kTile + (threadIdx.x & 63)));
+        update_mixed_at_once<S, XOPEN, NT>(a, t, w, j, k, a.link + ((size_t)code * kTile + (threadIdx.x & 63)));
     } else {
         const uint32_t lm = a.link[(size_t)code * kTile + (threadIdx.x & 63)];
-        update_tile<S, XOPEN, true>(a, t, w, j, k, lm);
+        update_tile<S, XOPEN, NT, true>(a, t, w, j, k, lm);
     }
 }
 
 // No register target beyond the block size: asking the compiler for 8 wavefronts per SIMD (64
 // registers) makes it interleave the 19 loads with their uses and costs the 2-byte storages
 // 7-13 % on MI355X, although it removes only one register.
-template <typename S, bool XOPEN>
+template <typename S, bool XOPEN, bool NT>
 __global__ __launch_bounds__(kBlock) void k_fused(XArgs<S> a)
 {
-    fused_step<S, XOPEN>(a);
+    fused_step<S, XOPEN, NT>(a);
 }
 
 // e3m12 with open x faces, with a budget of 96 scalar registers (101 without): still seven
@@ -455,9 +449,9 @@ __global__ __launch_bounds__(kBlock) void k_fused(XArgs<S> a)
 // 7 %: there it lets an eighth wavefront in, whose extra 19 loads in flight per lane disorder the
 // memory request stream.
 template <>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_num_sgpr(96))) void k_fused<e3m12_t, true>(XArgs<e3m12_t> a)
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_num_sgpr(96))) void k_fused<e3m12_t, true, true>(XArgs<e3m12_t> a)
 {
-    fused_step<e3m12_t, true>(a);
+    fused_step<e3m12_t, true, true>(a);
 }
 
 // FP64 with open x faces, compiled for the three wavefronts per SIMD that its block cap allows:
@@ -465,9 +459,9 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_num_sgpr(96))) void k
 // instead of 1.637 ms per 512 x 256 x 256 sponge step on MI355X (the parity stream-collide under
 // the same hint: no change).
 template <>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(1, 3))) void k_fused<double, true>(XArgs<double> a)
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(1, 3))) void k_fused<double, true, true>(XArgs<double> a)
 {
-    fused_step<double, true>(a);
+    fused_step<double, true, true>(a);
 }
 
 #include "eup_pair.h"
@@ -745,9 +739,28 @@ static int fused_block_order(const Handle *h, int cap)
     return window >= plane ? 2 : 1;
 }
 
+// bytes of the two state buffers
+template <typename S> double two_states(const Handle *h)
+{
+    return 2.0 * sizeof(S) * kTileElems * (double)h->g.tiles;
+}
+
 static size_t fused_lds_bytes(const Handle *h) { return occupancy_lds_bytes(h, fused_cap(h)); }
 
 } // namespace
+
+// Whether a step's stores go past the caches (non-temporal).  They do not where the two state buffers
+// stay in the 256 MB memory-side cache from step to step, down to the 32 MB of the L2 caches.  us per
+// step, non-temporal against cached, without obstacles (MB of the two buffers): FP64 128 x 64 x 64 (159)
+// 30.3 / 25.7, 128 x 128 x 64 (319) 55.3 / 56.7, 192 x 96 x 96 (538) 89.7 / 99.2; FP32 64 x 64 x 64
+// (40) 8.4 / 9.3, 128 x 64 x 64 (80) 16.3 / 14.1, 192 x 96 x 96 (269) 47.2 / 43.0 (two steps per launch
+// 39.1 / 36.6), 256 x 128 x 64 (319) 54.8 / 53.8 (44.8 / 46.5); FP16 256 x 128 x 64 (159) 29.1 / 26.9, 256 x
+// 128 x 128 (319) 54.2 / 52.8, but BF16 there with an obstacle 97.0 / 99.6.  EUP_CACHED_STORES=0 / 1 forces either.
+bool stream_stores(const Handle *h, double bytes)
+{
+    if (const char *e = getenv("EUP_CACHED_STORES")) return atoi(e) == 0;
+    return bytes < 50e6 || bytes > 280e6;
+}
 
 // dynamic LDS per block that limits a kernel without LDS to `cap` blocks per CU (0 = no limit)
 size_t occupancy_lds_bytes(const Handle *h, int cap)
@@ -767,6 +780,7 @@ size_t occupancy_lds_bytes(const Handle *h, int cap)
 
 namespace {
 
+
 template <typename S> int step_t(Handle *h)
 {
     if (h->fused_remap < 0) h->fused_remap = fused_block_order(h, fused_cap(h));
@@ -774,10 +788,15 @@ template <typename S> int step_t(Handle *h)
     const unsigned grid = 8u * a.chunk; // multiple of 8 so the XCD remap is a bijection
     if (h->fused_lds == (size_t)-1) h->fused_lds = fused_lds_bytes(h);
     const size_t lds = h->fused_lds;
-    if (x_open(h))
-        hipLaunchKernelGGL((k_fused<S, true>), dim3(grid), dim3(kBlock), lds, h->stream, a);
-    else
-        hipLaunchKernelGGL((k_fused<S, false>), dim3(grid), dim3(kBlock), lds, h->stream, a);
+    auto launch = [&](auto nt) {
+        constexpr bool NT = decltype(nt)::value;
+        if (x_open(h))
+            hipLaunchKernelGGL((k_fused<S, true, NT>), dim3(grid), dim3(kBlock), lds, h->stream, a);
+        else
+            hipLaunchKernelGGL((k_fused<S, false, NT>), dim3(grid), dim3(kBlock), lds, h->stream, a);
+    };
+    if (stream_stores(h, two_states<S>(h))) launch(std::true_type{});
+    else launch(std::false_type{});
     if (hip_check(h, hipGetLastError(), "fused step launch")) return EUP_EHIP;
     h->cur ^= 1;
     return 0;
@@ -823,10 +842,11 @@ template <typename S> PairMap pair_map(const Handle *h, double *us)
 
 // Whether the handle's steps are taken two per launch: where a pair is expected to be at least a tenth
 // faster than two single steps (columns with obstacles cost a pair up to that much more), these at the
-// 6.1 TB/s and 2.5 us per launch that they reach.  Measured, single against pair per step, without
-// obstacles: FP32 64 x 64 x 64 8.5 / 10.1 us (single), 128 x 64 x 64 16.2 / 14.6, 256 x 128 x 128
-// 105 / 82, 680 x 340 x 4 27.3 / 30.8 (single), 512 x 256 x 256 813 / 571; FP64 128 x 64 x 64 30.3 / 30.5
-// (single), 256 x 128 x 128 210 / 178, 512 x 256 x 256 1659 / 1285.
+// 6.1 TB/s and 2.5 us per launch that they reach (0.5 us with cached stores).  Measured, single
+// against pair per step, without obstacles: FP32 64 x 64 x 64 8.5 / 10.1 us (single), 128 x 64 x 64
+// 14.1 / 14.7 (single), 170 x 77 x 51 20.0 / 18.7, 256 x 128 x 128 105 / 82, 680 x 340 x 4 27.3 / 30.8 (single),
+// 512 x 256 x 256 813 / 571; FP64 128 x 64 x 64 25.7 / 28.8 (single), 256 x 128 x 128 210 / 178,
+// 512 x 256 x 256 1659 / 1285.
 template <typename S> bool pair_better(const Handle *h)
 {
     const Geometry &g = h->g;
@@ -836,20 +856,20 @@ template <typename S> bool pair_better(const Handle *h)
     if (const char *e = getenv("EUP_PAIR")) return atoi(e) != 0;
     double us;
     pair_map<S>(h, &us);
-    return 1.1 * us < 2.0 * (2.5 + (double)g.tiles * (2 * kTileElems * sizeof(S)) / 6.1e6);
+    return 1.1 * us < 2.0 * ((stream_stores(h, two_states<S>(h)) ? 2.5 : 0.5) + two_states<S>(h) / 6.1e6);
 }
 
-template <typename S, bool XOPEN> int pair_launches(Handle *h, int count)
+template <typename S, bool XOPEN, bool NT> int pair_launches(Handle *h, int count)
 {
     const size_t lds = pair_lds_bytes<S>();
-    if (hip_check(h, hipFuncSetAttribute(reinterpret_cast<const void *>(k_pair<S, XOPEN>),
+    if (hip_check(h, hipFuncSetAttribute(reinterpret_cast<const void *>(k_pair<S, XOPEN, NT>),
                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds), "two-step LDS"))
         return EUP_EHIP;
     double us;
     const PairMap pm = pair_map<S>(h, &us);
     for (int i = 0; i < count; ++i) {
         const XArgs<S> a = make_args<S>(h);
-        hipLaunchKernelGGL((k_pair<S, XOPEN>), dim3(pm.blocks), dim3(pair_threads<S>()), lds, h->stream, a, pm);
+        hipLaunchKernelGGL((k_pair<S, XOPEN, NT>), dim3(pm.blocks), dim3(pair_threads<S>()), lds, h->stream, a, pm);
         if (hip_check(h, hipGetLastError(), "two-step launch")) return EUP_EHIP;
         h->cur ^= 1;
     }
@@ -912,7 +932,11 @@ int physics_steps(Handle *h, int nsteps)
         int t = 0, rc = 0;
         if constexpr (kPairs<S>) {
             if (nsteps > 1 && pair_better<S>(h)) {
-                rc = x_open(h) ? pair_launches<S, true>(h, nsteps / 2) : pair_launches<S, false>(h, nsteps / 2);
+                auto launches = [&](auto nt) {
+                    constexpr bool NT = decltype(nt)::value;
+                    return x_open(h) ? pair_launches<S, true, NT>(h, nsteps / 2) : pair_launches<S, false, NT>(h, nsteps / 2);
+                };
+                rc = stream_stores(h, two_states<S>(h)) ? launches(std::true_type{}) : launches(std::false_type{});
                 t = nsteps / 2 * 2;
             }
         }
