@@ -109,17 +109,40 @@ static void release(Handle *h)
 {
     if (!h) return;
     if (h->stream) hipStreamSynchronize(h->stream);
-    void *ptrs[] = {h->alloc[0], h->alloc[1], h->staging, h->obs_stage, h->solid, h->solid_list, h->bb_tmp,
+    void *ptrs[] = {h->alloc[0], h->alloc[1], h->obs_stage, h->solid, h->solid_list, h->bb_tmp,
                     h->tile_code, h->link_mask, h->mixed_list, h->outlet[0], h->outlet[1], h->diag,
                     h->site19, h->grey, h->grey_zero, h->work};
     for (void *p : ptrs)
         if (p) hipFree(p);
+    if (h->pinned) hipHostFree(h->pinned);
+    for (hipEvent_t e : h->moved)
+        if (e) hipEventDestroy(e);
     if (h->ev0) hipEventDestroy(h->ev0);
     if (h->ev1) hipEventDestroy(h->ev1);
     if (h->stream) hipStreamDestroy(h->stream);
 }
 
 namespace eup {
+
+int transfer_ready(Handle *h, int64_t bytes)
+{
+    for (hipEvent_t &e : h->moved)
+        if (!e && hip_check(h, hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate")) {
+            e = nullptr;
+            return EUP_EHIP;
+        }
+    if (h->pinned_len >= bytes) return 0;
+    if (h->pinned) hipHostFree(h->pinned);
+    h->pinned = nullptr;
+    h->pinned_len = 0;
+    if (hip_check(h, hipHostMalloc((void **)&h->pinned, (size_t)bytes), "hipHostMalloc transfer")) {
+        h->pinned = nullptr;
+        return EUP_EHIP;
+    }
+    h->pinned_len = bytes;
+    return 0;
+}
+
 namespace {
 
 // sites of one chunk of the obstacle list marked solid (indices validated on the host)
@@ -242,9 +265,7 @@ int eup_create(const eup_config *cfg, eup_handle **out)
     // defined contents in the guard tiles and the padding lanes of partial tiles
     for (int b = 0; b < 2 && !rc && h->tiled; ++b)
         if (hip_check(h, hipMemset(h->alloc[b], 0, state), "hipMemset populations")) rc = EUP_EHIP;
-    if (!rc && (hip_check(h, hipMalloc((void **)&h->staging, sizeof(double) * g.ghosted), "hipMalloc staging") ||
-                hip_check(h, hipMalloc((void **)&h->solid, g.sites), "hipMalloc solid")))
-        rc = EUP_EHIP;
+    if (!rc && hip_check(h, hipMalloc((void **)&h->solid, g.sites), "hipMalloc solid")) rc = EUP_EHIP;
     if (!rc && cfg->mode == EUP_MODE_PHYSICS) {
         const size_t rb = cfg->storage == EUP_STORE_F64 ? 8 : 4;
         for (int b = 0; b < 2 && !rc; ++b)
@@ -267,7 +288,7 @@ int eup_create(const eup_config *cfg, eup_handle **out)
     const size_t outlet = cfg->mode == EUP_MODE_PHYSICS
                               ? 2 * (cfg->storage == EUP_STORE_F64 ? 8 : 4) * 5 * (size_t)g.m * g.n
                               : (cfg->mode == EUP_MODE_PARITY ? sizeof(double) * 5 * (size_t)g.m * g.n : 0);
-    h->device_bytes = (int64_t)(2 * state + sizeof(double) * g.ghosted + g.sites + outlet);
+    h->device_bytes = (int64_t)(2 * state + g.sites + outlet);
     *out = h;
     return 0;
 }
@@ -423,34 +444,34 @@ static int check_q(eup_handle *h, int32_t q)
     return 0;
 }
 
+static int set_pops(eup_handle *h, int q, int nq, const double *a)
+{
+    if (hip_check(h, hipSetDevice(h->cfg.device), "hipSetDevice")) return EUP_EHIP;
+    h->outlet_dirty = true;
+    int rc = h->cfg.mode == EUP_MODE_PARITY ? parity_set_pops(h, q, nq, a) : physics_set_pops(h, q, nq, a);
+    if (rc) return rc;
+    h->pops_set |= ((1u << nq) - 1) << q;
+    return 0;
+}
+
+static int get_pops(eup_handle *h, int q, int nq, double *a)
+{
+    if (hip_check(h, hipSetDevice(h->cfg.device), "hipSetDevice")) return EUP_EHIP;
+    return h->cfg.mode == EUP_MODE_PARITY ? parity_get_pops(h, q, nq, a) : physics_get_pops(h, q, nq, a);
+}
+
 int eup_set_pops(eup_handle *h, int32_t q, const double *a)
 {
     if (!h || !a) return fail(h, EUP_EINVAL, "eup_set_pops: null argument");
     if (check_q(h, q)) return EUP_ERANGE;
-    if (hip_check(h, hipSetDevice(h->cfg.device), "hipSetDevice") ||
-        hip_check(h, hipMemcpyAsync(h->staging, a, sizeof(double) * h->g.ghosted, hipMemcpyHostToDevice,
-                                    h->stream), "copy pops"))
-        return EUP_EHIP;
-    int rc = h->cfg.mode == EUP_MODE_PARITY ? parity_set_pop(h, q) : physics_set_pop(h, q);
-    if (rc) return rc;
-    if (hip_check(h, hipStreamSynchronize(h->stream), "sync")) return EUP_EHIP;
-    h->outlet_dirty = true;
-    h->pops_set |= 1u << (q - 1);
-    return 0;
+    return set_pops(h, q - 1, 1, a);
 }
 
 int eup_get_pops(eup_handle *h, int32_t q, double *a)
 {
     if (!h || !a) return fail(h, EUP_EINVAL, "eup_get_pops: null argument");
     if (check_q(h, q)) return EUP_ERANGE;
-    if (hip_check(h, hipSetDevice(h->cfg.device), "hipSetDevice")) return EUP_EHIP;
-    int rc = h->cfg.mode == EUP_MODE_PARITY ? parity_get_pop(h, q) : physics_get_pop(h, q);
-    if (rc) return rc;
-    if (hip_check(h, hipMemcpyAsync(a, h->staging, sizeof(double) * h->g.ghosted, hipMemcpyDeviceToHost,
-                                    h->stream), "copy pops") ||
-        hip_check(h, hipStreamSynchronize(h->stream), "sync"))
-        return EUP_EHIP;
-    return 0;
+    return get_pops(h, q - 1, 1, a);
 }
 
 int eup_init_equilibrium(eup_handle *h, double ux, double uy, double uz, double noise, uint64_t seed)
@@ -468,21 +489,13 @@ int eup_init_equilibrium(eup_handle *h, double ux, double uy, double uz, double 
 int eup_set_state(eup_handle *h, const double *a)
 {
     if (!h || !a) return fail(h, EUP_EINVAL, "eup_set_state: null argument");
-    for (int q = 1; q <= 19; ++q) {
-        int rc = eup_set_pops(h, q, a + (int64_t)(q - 1) * h->g.ghosted);
-        if (rc) return rc;
-    }
-    return 0;
+    return set_pops(h, 0, 19, a);
 }
 
 int eup_get_state(eup_handle *h, double *a)
 {
     if (!h || !a) return fail(h, EUP_EINVAL, "eup_get_state: null argument");
-    for (int q = 1; q <= 19; ++q) {
-        int rc = eup_get_pops(h, q, a + (int64_t)(q - 1) * h->g.ghosted);
-        if (rc) return rc;
-    }
-    return 0;
+    return get_pops(h, 0, 19, a);
 }
 
 static int ready(eup_handle *h, const char *who)

@@ -12,6 +12,7 @@
 #include <vector>
 
 #include "eup_internal.h"
+#include "eup_transfer.h"
 
 // Device scratch of eup_drag_cv_noalloc: the per-site stresses of the two faces of one axis,
 // at most kNoAllocFace sites per face (16 MiB per GPU, held for the life of the process).  Host
@@ -243,36 +244,55 @@ __device__ __forceinline__ void vtk_site(const Acc &acc, int i, int j, int k, fl
     o[2] = v / den;
 }
 
-// one plane of velocities in the writers' loop order: plane 0 = yz at x = index (k, j), 1 = xz at
-// y = index (k, i), 2 = xy at z = index (j, i)
+// `count` velocities from site t0 on of a plane in the writers' loop order, into pinned host memory:
+// plane 0 = yz at x = index (k, j), 1 = xz at y = index (k, i), 2 = xy at z = index (j, i), 3 = the
+// lattice (k, j, i).  The block's 3 x 256 floats go through LDS, so that what crosses the bus is whole
+// lines.
 template <typename Acc>
-__global__ void k_vtk_velocity(Acc acc, int plane, int index, float *out)
+__global__ __launch_bounds__(kBlock) void k_vtk_velocity(Acc acc, int plane, int index, int64_t t0, int64_t count,
+                                                         float *out)
 {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int l = acc.l, m = acc.m, n = acc.n;
-    int i, j, k;
-    if (plane == 0) {
-        if (t >= (int64_t)m * n) return;
-        i = index; j = 1 + (int)(t % m); k = 1 + (int)(t / m);
-    } else if (plane == 1) {
-        if (t >= (int64_t)l * n) return;
-        i = 1 + (int)(t % l); j = index; k = 1 + (int)(t / l);
-    } else {
-        if (t >= (int64_t)l * m) return;
-        i = 1 + (int)(t % l); j = 1 + (int)(t / l); k = index;
+    __shared__ __align__(16) float sh[3 * kBlock];
+    const int64_t b0 = (int64_t)blockIdx.x * kBlock;
+    const int nb = (int)(count - b0 < kBlock ? count - b0 : kBlock);
+    if ((int)threadIdx.x < nb) {
+        const int64_t t = t0 + b0 + threadIdx.x;
+        const uint32_t w = plane == 0 ? acc.m : acc.l; // the fastest coordinate's extent
+        const uint64_t r = (uint64_t)t / w;
+        const int u = 1 + (int)((uint64_t)t - r * w);
+        int i = u, j = index, k = index;
+        if (plane == 0) {
+            i = index; j = u; k = 1 + (int)r;
+        } else if (plane == 1) {
+            k = 1 + (int)r;
+        } else if (plane == 2) {
+            j = 1 + (int)r;
+        } else {
+            const uint64_t z = r / (uint32_t)acc.m;
+            j = 1 + (int)(r - z * (uint32_t)acc.m);
+            k = 1 + (int)z;
+        }
+        vtk_site(acc, i, j, k, sh + 3 * threadIdx.x);
     }
-    vtk_site(acc, i, j, k, out + 3 * t);
+    __syncthreads();
+    float *o = out + 3 * b0;
+    if (nb == kBlock) {
+        if (threadIdx.x < 3 * kBlock / 4)
+            reinterpret_cast<float4 *>(o)[threadIdx.x] = reinterpret_cast<const float4 *>(sh)[threadIdx.x];
+    } else {
+        for (int e = threadIdx.x; e < 3 * nb; e += kBlock) o[e] = sh[e];
+    }
 }
 
 // vorticity of the xy plane z = k0 as vtk_om.binary.F90:88-131 computes it (i = 2..l-1 fastest,
 // j = 2..m-1): densities rounded to float; in each momentum only the last population is divided
 // by the density, as the writer's expression reads; the difference is formed in float
 template <typename Acc>
-__global__ void k_vtk_vorticity(Acc acc, int k0, float *out)
+__global__ void k_vtk_vorticity(Acc acc, int k0, int64_t t0, int64_t count, float *out)
 {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int l = acc.l, m = acc.m;
-    if (t >= (int64_t)(l - 2) * (m - 2)) return;
+    const int64_t o = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, t = t0 + o;
+    const int l = acc.l;
+    if (o >= count) return;
     const int i = 2 + (int)(t % (l - 2)), j = 2 + (int)(t / (l - 2));
     const int di[4] = {0, 0, -1, 1}, dj[4] = {1, -1, 0, 0}; // up, down, left, right
     float mom[4];
@@ -288,7 +308,7 @@ __global__ void k_vtk_vorticity(Acc acc, int k0, float *out)
         else
             mom[s] = (float)(x[2] + x[6] + x[7] + x[8] + x[11] - x[0] - x[9] - x[15] - x[16] - x[17] / (double)d);
     }
-    out[t] = 0.5f * (mom[0] - mom[1]) - 0.5f * (mom[3] - mom[2]);
+    out[o] = 0.5f * (mom[0] - mom[1]) - 0.5f * (mom[3] - mom[2]);
 }
 
 template <typename Acc>
@@ -560,56 +580,30 @@ int diag_drag_mem(Handle *h, double F[3])
     return 0;
 }
 
-// one velocity plane into out (host), through a plane-sized device buffer
-static int vtk_plane(Handle *h, int plane, int index, float *out)
-{
-    const Geometry &g = h->g;
-    const int64_t count = plane == 0 ? (int64_t)g.m * g.n : (plane == 1 ? (int64_t)g.l * g.n : (int64_t)g.l * g.m);
-    int rc = ensure_diag(h, (3 * count + 1) / 2 + 1);
-    if (rc) return rc;
-    float *dev = reinterpret_cast<float *>(h->diag);
-    rc = with_acc(h, [&](auto acc) {
-        hipLaunchKernelGGL((k_vtk_velocity<decltype(acc)>), dim3((unsigned)((count + 255) / 256)), dim3(256), 0,
-                           h->stream, acc, plane, index, dev);
-        return hip_check(h, hipGetLastError(), "vtk velocity") ? EUP_EHIP : 0;
-    });
-    if (rc) return rc;
-    if (hip_check(h, hipMemcpyAsync(out, dev, sizeof(float) * 3 * count, hipMemcpyDeviceToHost, h->stream),
-                  "copy vtk") ||
-        hip_check(h, hipStreamSynchronize(h->stream), "sync"))
-        return EUP_EHIP;
-    return 0;
-}
-
 int diag_vtk_velocity(Handle *h, int plane, int index, float *out)
 {
-    if (plane != 3) return vtk_plane(h, plane, index, out);
-    // the volume in the writer's order (k, j, i) = the xy planes one after the other
-    const int64_t per = (int64_t)h->g.l * h->g.m * 3;
-    for (int k = 1; k <= h->g.n; ++k) {
-        int rc = vtk_plane(h, 2, k, out + (k - 1) * per);
-        if (rc) return rc;
-    }
-    return 0;
+    const Geometry &g = h->g;
+    const int64_t count = plane == 0   ? (int64_t)g.m * g.n
+                          : plane == 1 ? (int64_t)g.l * g.n
+                          : plane == 2 ? (int64_t)g.l * g.m
+                                       : g.sites;
+    return with_acc(h, [&](auto acc) {
+        return transfer<false>(h, (char *)out, 12 * count, 12 * kBlock, [=](int64_t at, int64_t len, char *pinned) {
+            hipLaunchKernelGGL((k_vtk_velocity<decltype(acc)>), dim3((unsigned)((len / 12 + kBlock - 1) / kBlock)),
+                               dim3(kBlock), 0, h->stream, acc, plane, index, at / 12, len / 12, (float *)pinned);
+        });
+    });
 }
 
 int diag_vtk_vorticity(Handle *h, int k0, float *out)
 {
     const int64_t count = (int64_t)(h->g.l - 2) * (h->g.m - 2);
-    int rc = ensure_diag(h, count / 2 + 1);
-    if (rc) return rc;
-    float *dev = reinterpret_cast<float *>(h->diag);
-    rc = with_acc(h, [&](auto acc) {
-        hipLaunchKernelGGL((k_vtk_vorticity<decltype(acc)>), dim3((unsigned)((count + 255) / 256)), dim3(256), 0,
-                           h->stream, acc, k0, dev);
-        return hip_check(h, hipGetLastError(), "vtk vorticity") ? EUP_EHIP : 0;
+    return with_acc(h, [&](auto acc) {
+        return transfer<false>(h, (char *)out, 4 * count, 4, [=](int64_t at, int64_t len, char *pinned) {
+            hipLaunchKernelGGL((k_vtk_vorticity<decltype(acc)>), dim3((unsigned)((len / 4 + 255) / 256)), dim3(256), 0,
+                               h->stream, acc, k0, at / 4, len / 4, (float *)pinned);
+        });
     });
-    if (rc) return rc;
-    if (hip_check(h, hipMemcpyAsync(out, dev, sizeof(float) * count, hipMemcpyDeviceToHost, h->stream),
-                  "copy vtk") ||
-        hip_check(h, hipStreamSynchronize(h->stream), "sync"))
-        return EUP_EHIP;
-    return 0;
 }
 
 int diag_diagno(Handle *h, double out[5])

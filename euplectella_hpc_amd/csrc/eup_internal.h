@@ -41,7 +41,6 @@ struct Handle {
     void *alloc[2] = {nullptr, nullptr}; // device allocations of the two state buffers
     void *buf[2] = {nullptr, nullptr}; // ping-pong population buffers (past the leading guard)
     int cur = 0;                  // buf[cur] holds the current state
-    double *staging = nullptr;    // ghosted FP64 staging array (one population)
     bool mask_set = false;
     uint32_t pops_set = 0;        // bit q-1 set once population q has been provided
     // mask derived data
@@ -74,6 +73,9 @@ struct Handle {
     bool grey_set = false;
     void *work = nullptr;         // objective scratch kept between calls
     size_t work_len = 0;
+    char *pinned = nullptr;       // pinned pieces of transfers to and from the host
+    int64_t pinned_len = 0;
+    hipEvent_t moved[8] = {};     // per piece: its kernel has run
     int64_t device_bytes = 0;
 };
 
@@ -90,11 +92,12 @@ int parity_step(Handle *h);
 int physics_prepare_mask(Handle *h);
 int physics_steps(Handle *h, int nsteps);
 int physics_refresh_outlet(Handle *h);
-int physics_set_pop(Handle *h, int q); // staging (ghosted f64) -> both buffers
-int physics_get_pop(Handle *h, int q); // current buffer -> staging
-int parity_set_pop(Handle *h, int q);
+// nq populations from q (0-based) on between the reference's ghosted FP64 arrays and the state
+int physics_set_pops(Handle *h, int q, int nq, const double *a); // -> both buffers
+int physics_get_pops(Handle *h, int q, int nq, double *a);
+int parity_set_pops(Handle *h, int q, int nq, const double *a);
+int parity_get_pops(Handle *h, int q, int nq, double *a);
 int init_equilibrium(Handle *h, double ux, double uy, double uz, double noise, uint64_t seed);
-int parity_get_pop(Handle *h, int q);
 
 // grey mode (eup_grey.hip)
 // bytes of a grey state: 19 populations and the outlet ghost plane

@@ -21,6 +21,7 @@
 #include <stdlib.h>
 
 #include "eup_internal.h"
+#include "eup_transfer.h"
 
 namespace eup {
 
@@ -269,28 +270,27 @@ template <bool NT> __global__ __launch_bounds__(256) void k_stream_collide(PArgs
     }
 }
 
-// one population between the reference's ghosted array (row pitch l + 2; the staging buffer) and
-// the padded layout (row pitch `pitch`), ghosted site t = i + (l+2) (j + (m+2) k)
-__global__ void k_parity_put(const double *__restrict__ stg, double *__restrict__ d0, double *__restrict__ d1,
-                             int l, int m, int n, int pitch)
+// `count` elements from element t0 on of the reference's ghosted arrays (row pitch l + 2, one population
+// after the other), in pinned host memory, into both buffers
+__global__ void k_parity_put(const double *__restrict__ a, int64_t t0, int64_t count, double *__restrict__ d0,
+                             double *__restrict__ d1, int l, int64_t rows, int pitch, int64_t stride)
 {
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= (int64_t)(l + 2) * (m + 2) * (n + 2)) return;
-    const int i = (int)(t % (l + 2));
-    const int64_t r = t / (l + 2);
-    const int64_t e = i + (int64_t)pitch * r;
-    d0[e] = stg[t];
-    d1[e] = stg[t];
+    if (t >= count) return;
+    const int64_t row = (t0 + t) / (l + 2), q = row / rows;
+    const int64_t e = (t0 + t) - row * (l + 2) + pitch * (row - q * rows) + q * stride;
+    d0[e] = a[t];
+    d1[e] = a[t];
 }
 
-__global__ void k_parity_take(const double *__restrict__ src, double *__restrict__ stg, int l, int m, int n,
-                              int pitch)
+// ... and back
+__global__ void k_parity_take(const double *__restrict__ src, double *__restrict__ a, int64_t t0, int64_t count,
+                              int l, int64_t rows, int pitch, int64_t stride)
 {
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= (int64_t)(l + 2) * (m + 2) * (n + 2)) return;
-    const int i = (int)(t % (l + 2));
-    const int64_t r = t / (l + 2);
-    stg[t] = src[i + (int64_t)pitch * r];
+    if (t >= count) return;
+    const int64_t row = (t0 + t) / (l + 2), q = row / rows;
+    a[t] = src[(t0 + t) - row * (l + 2) + pitch * (row - q * rows) + q * stride];
 }
 
 PArgs make_args(Handle *h, int from)
@@ -417,23 +417,26 @@ int parity_step(Handle *h)
     return 0;
 }
 
-int parity_set_pop(Handle *h, int q)
+int parity_set_pops(Handle *h, int q, int nq, const double *a)
 {
     const Geometry &g = h->g;
-    double *d0 = static_cast<double *>(h->buf[0]) + (int64_t)(q - 1) * h->stride + h->poff;
-    double *d1 = static_cast<double *>(h->buf[1]) + (int64_t)(q - 1) * h->stride + h->poff;
-    hipLaunchKernelGGL(k_parity_put, dim3(nblocks(g.ghosted, 256)), dim3(256), 0, h->stream, h->staging, d0, d1,
-                       g.l, g.m, g.n, h->ppitch);
-    return hip_check(h, hipGetLastError(), "set pops") ? EUP_EHIP : 0;
+    const int64_t t0 = q * g.ghosted, rows = (int64_t)(g.m + 2) * (g.n + 2);
+    return transfer<true>(h, (char *)a, 8 * nq * g.ghosted, 8, [=](int64_t at, int64_t len, char *pinned) {
+        hipLaunchKernelGGL(k_parity_put, dim3(nblocks(len / 8, 256)), dim3(256), 0, h->stream, (const double *)pinned,
+                           t0 + at / 8, len / 8, static_cast<double *>(h->buf[0]) + h->poff,
+                           static_cast<double *>(h->buf[1]) + h->poff, h->g.l, rows, h->ppitch, h->stride);
+    });
 }
 
-int parity_get_pop(Handle *h, int q)
+int parity_get_pops(Handle *h, int q, int nq, double *a)
 {
     const Geometry &g = h->g;
-    const double *src = static_cast<const double *>(h->buf[h->cur]) + (int64_t)(q - 1) * h->stride + h->poff;
-    hipLaunchKernelGGL(k_parity_take, dim3(nblocks(g.ghosted, 256)), dim3(256), 0, h->stream, src, h->staging,
-                       g.l, g.m, g.n, h->ppitch);
-    return hip_check(h, hipGetLastError(), "get pops") ? EUP_EHIP : 0;
+    const int64_t t0 = q * g.ghosted, rows = (int64_t)(g.m + 2) * (g.n + 2);
+    return transfer<false>(h, (char *)a, 8 * nq * g.ghosted, 8, [=](int64_t at, int64_t len, char *pinned) {
+        hipLaunchKernelGGL(k_parity_take, dim3(nblocks(len / 8, 256)), dim3(256), 0, h->stream,
+                           static_cast<const double *>(h->buf[h->cur]) + h->poff, (double *)pinned, t0 + at / 8,
+                           len / 8, h->g.l, rows, h->ppitch, h->stride);
+    });
 }
 
 } // namespace eup

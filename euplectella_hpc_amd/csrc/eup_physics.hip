@@ -30,6 +30,7 @@
 #include <type_traits>
 
 #include "eup_internal.h"
+#include "eup_transfer.h"
 
 namespace eup {
 
@@ -539,35 +540,42 @@ __global__ void k_compact_links(const int32_t *__restrict__ code, const uint32_t
 // ---------------------------------------------------------------------------------------------
 // state conversion and outlet refresh
 // ---------------------------------------------------------------------------------------------
-template <typename S>
-__global__ void k_from_staging(const double *__restrict__ stg, S *__restrict__ d0, S *__restrict__ d1,
-                               PopIndex P, int l, int m, int n, int q, float ref)
+// element t of consecutive ghosted arrays (l + 2, m + 2, n + 2) from population 0 on: its population
+// and 0-based site; false on the ghost shell
+__device__ __forceinline__ bool ghosted_site(int64_t t, int l, int m, int n, int &q, int &i, int &j, int &k)
 {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t N = (int64_t)l * m * n;
-    if (t >= N) return;
-    const int i = (int)(t % l);
-    const int64_t r = t / l;
-    const int j = (int)(r % m), k = (int)(r / m);
-    const double v = stg[(int64_t)(i + 1) + (int64_t)(l + 2) * ((int64_t)(j + 1) + (int64_t)(m + 2) * (k + 1))];
-    const S sv = Store<S>::store64(v, ref, q);
-    const int64_t e = P(q, i, j, k);
-    d0[e] = sv;
-    d1[e] = sv;
+    const uint32_t L = (uint32_t)l + 2, M = (uint32_t)m + 2, N = (uint32_t)n + 2;
+    const uint64_t r = (uint64_t)t / L, p = r / M;
+    i = (int)((uint64_t)t - r * L) - 1;
+    j = (int)(r - p * M) - 1;
+    q = (int)(p / N);
+    k = (int)(p - (uint64_t)q * N) - 1;
+    return (uint32_t)i < (uint32_t)l && (uint32_t)j < (uint32_t)m && (uint32_t)k < (uint32_t)n;
 }
 
+// `count` elements from element t0 of the ghosted arrays, the arrays in pinned host memory
 template <typename S>
-__global__ void k_to_staging(const S *__restrict__ src, double *__restrict__ stg, PopIndex P, int l, int m,
-                             int n, int q, float ref)
+__global__ void k_pops_in(const double *__restrict__ a, int64_t t0, int64_t count, S *__restrict__ d0,
+                          S *__restrict__ d1, PopIndex P, int l, int m, int n, DevRef ref)
 {
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t N = (int64_t)l * m * n;
-    if (t >= N) return;
-    const int i = (int)(t % l);
-    const int64_t r = t / l;
-    const int j = (int)(r % m), k = (int)(r / m);
-    stg[(int64_t)(i + 1) + (int64_t)(l + 2) * ((int64_t)(j + 1) + (int64_t)(m + 2) * (k + 1))] =
-        Store<S>::load64(src[P(q, i, j, k)], ref, q);
+    int q, i, j, k;
+    if (t >= count || !ghosted_site(t0 + t, l, m, n, q, i, j, k)) return;
+    const S v = Store<S>::store64(a[t], ref.r[q], q);
+    const int64_t e = P(q, i, j, k);
+    d0[e] = v;
+    d1[e] = v;
+}
+
+// ... and back, the ghost shell as zeros
+template <typename S>
+__global__ void k_pops_out(const S *__restrict__ src, double *__restrict__ a, int64_t t0, int64_t count, PopIndex P,
+                           int l, int m, int n, DevRef ref)
+{
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= count) return;
+    int q, i, j, k;
+    a[t] = ghosted_site(t0 + t, l, m, n, q, i, j, k) ? Store<S>::load64(src[P(q, i, j, k)], ref.r[q], q) : 0.0;
 }
 
 // counter-based uniform in [-1, 1) (splitmix64 finaliser)
@@ -894,25 +902,24 @@ template <typename S> int refresh_t(Handle *h)
     return hip_check(h, hipGetLastError(), "outlet refresh") ? EUP_EHIP : 0;
 }
 
-template <typename S> int set_t(Handle *h, int q)
+template <typename S> int set_t(Handle *h, int q, int nq, const double *a)
 {
-    S *d0 = static_cast<S *>(h->buf[0]);
-    S *d1 = static_cast<S *>(h->buf[1]);
-    hipLaunchKernelGGL((k_from_staging<S>), dim3((unsigned)((h->g.sites + 255) / 256)), dim3(256), 0,
-                       h->stream, h->staging, d0, d1, pop_index(h), h->g.l, h->g.m, h->g.n, q - 1,
-                       dev_ref(h).r[q - 1]);
-    return hip_check(h, hipGetLastError(), "set pops") ? EUP_EHIP : 0;
+    const int64_t t0 = (int64_t)q * h->g.ghosted;
+    return transfer<true>(h, (char *)a, 8 * nq * h->g.ghosted, 8, [=](int64_t at, int64_t len, char *pinned) {
+        hipLaunchKernelGGL((k_pops_in<S>), dim3((unsigned)((len / 8 + 255) / 256)), dim3(256), 0, h->stream,
+                           (const double *)pinned, t0 + at / 8, len / 8, static_cast<S *>(h->buf[0]),
+                           static_cast<S *>(h->buf[1]), pop_index(h), h->g.l, h->g.m, h->g.n, dev_ref(h));
+    });
 }
 
-template <typename S> int get_t(Handle *h, int q)
+template <typename S> int get_t(Handle *h, int q, int nq, double *a)
 {
-    const S *s = static_cast<const S *>(h->buf[h->cur]);
-    if (hip_check(h, hipMemsetAsync(h->staging, 0, sizeof(double) * h->g.ghosted, h->stream), "memset"))
-        return EUP_EHIP;
-    hipLaunchKernelGGL((k_to_staging<S>), dim3((unsigned)((h->g.sites + 255) / 256)), dim3(256), 0,
-                       h->stream, s, h->staging, pop_index(h), h->g.l, h->g.m, h->g.n, q - 1,
-                       dev_ref(h).r[q - 1]);
-    return hip_check(h, hipGetLastError(), "get pops") ? EUP_EHIP : 0;
+    const int64_t t0 = (int64_t)q * h->g.ghosted;
+    return transfer<false>(h, (char *)a, 8 * nq * h->g.ghosted, 8, [=](int64_t at, int64_t len, char *pinned) {
+        hipLaunchKernelGGL((k_pops_out<S>), dim3((unsigned)((len / 8 + 255) / 256)), dim3(256), 0, h->stream,
+                           static_cast<const S *>(h->buf[h->cur]), (double *)pinned, t0 + at / 8, len / 8,
+                           pop_index(h), h->g.l, h->g.m, h->g.n, dev_ref(h));
+    });
 }
 
 template <typename F> int dispatch(Handle *h, F &&f)
@@ -959,15 +966,14 @@ int physics_refresh_outlet(Handle *h)
     return dispatch(h, [&](auto *p) { return refresh_t<std::remove_pointer_t<decltype(p)>>(h); });
 }
 
-int physics_set_pop(Handle *h, int q)
+int physics_set_pops(Handle *h, int q, int nq, const double *a)
 {
-    h->outlet_dirty = true;
-    return dispatch(h, [&](auto *p) { return set_t<std::remove_pointer_t<decltype(p)>>(h, q); });
+    return dispatch(h, [&](auto *p) { return set_t<std::remove_pointer_t<decltype(p)>>(h, q, nq, a); });
 }
 
-int physics_get_pop(Handle *h, int q)
+int physics_get_pops(Handle *h, int q, int nq, double *a)
 {
-    return dispatch(h, [&](auto *p) { return get_t<std::remove_pointer_t<decltype(p)>>(h, q); });
+    return dispatch(h, [&](auto *p) { return get_t<std::remove_pointer_t<decltype(p)>>(h, q, nq, a); });
 }
 
 int init_equilibrium(Handle *h, double ux, double uy, double uz, double noise, uint64_t seed)
