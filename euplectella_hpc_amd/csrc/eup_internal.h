@@ -51,7 +51,6 @@ struct Handle {
     int32_t bbox[6] = {0, 0, 0, 0, 0, 0};
     // parity mode
     int32_t *solid_list = nullptr; // ghosted linear offsets of solid sites
-    double *bb_tmp = nullptr;      // nsolid x 18 bounce-back values
     // physics mode
     int32_t *tile_code = nullptr;  // per tile: kTileFluid, kTileSolid or index into link_mask
     uint32_t *link_mask = nullptr; // per mixed tile: 64 link masks
