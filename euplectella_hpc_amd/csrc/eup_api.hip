@@ -124,13 +124,8 @@ static void release(Handle *h)
 
 namespace eup {
 
-int transfer_ready(Handle *h, int64_t bytes)
+int pinned_ready(Handle *h, int64_t bytes)
 {
-    for (hipEvent_t &e : h->moved)
-        if (!e && hip_check(h, hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate")) {
-            e = nullptr;
-            return EUP_EHIP;
-        }
     if (h->pinned_len >= bytes) return 0;
     if (h->pinned) hipHostFree(h->pinned);
     h->pinned = nullptr;
@@ -141,6 +136,16 @@ int transfer_ready(Handle *h, int64_t bytes)
     }
     h->pinned_len = bytes;
     return 0;
+}
+
+int transfer_ready(Handle *h, int64_t bytes)
+{
+    for (hipEvent_t &e : h->moved)
+        if (!e && hip_check(h, hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate")) {
+            e = nullptr;
+            return EUP_EHIP;
+        }
+    return pinned_ready(h, bytes);
 }
 
 namespace {
@@ -399,18 +404,13 @@ int eup_commit_obstacles(eup_handle *h)
     h->mask_set = false; // set again only once the mask tables are rebuilt
     if (!h->obstacles_open && hip_check(h, hipMemsetAsync(h->solid, 0, g.sites, h->stream), "hipMemset solid"))
         return EUP_EHIP;
-    int64_t *part = nullptr, *part_h = nullptr;
-    int rc = 0;
-    if (hip_check(h, hipMalloc((void **)&part, sizeof(int64_t) * 8 * kStatBlocks), "hipMalloc") ||
-        hip_check(h, hipHostMalloc((void **)&part_h, sizeof(int64_t) * 8 * kStatBlocks), "hipHostMalloc"))
-        rc = EUP_EHIP;
+    // the blocks' results go straight to pinned memory
+    int rc = pinned_ready(h, sizeof(int64_t) * 8 * kStatBlocks);
+    const int64_t *part_h = reinterpret_cast<const int64_t *>(h->pinned);
     if (!rc) {
         hipLaunchKernelGGL(k_mask_stats, dim3(kStatBlocks), dim3(256), 0, h->stream, h->solid, g.l, g.m, g.sites,
-                           part);
-        if (hip_check(h, hipGetLastError(), "mask stats") ||
-            hip_check(h, hipMemcpyAsync(part_h, part, sizeof(int64_t) * 8 * kStatBlocks, hipMemcpyDeviceToHost,
-                                        h->stream), "copy stats") ||
-            hip_check(h, hipStreamSynchronize(h->stream), "sync"))
+                           reinterpret_cast<int64_t *>(h->pinned));
+        if (hip_check(h, hipGetLastError(), "mask stats") || hip_check(h, hipStreamSynchronize(h->stream), "sync"))
             rc = EUP_EHIP;
     }
     if (!rc) {
@@ -428,8 +428,6 @@ int eup_commit_obstacles(eup_handle *h)
         h->nsolid = ns;
         memcpy(h->bbox, bb, sizeof bb);
     }
-    hipFree(part);
-    if (part_h) hipHostFree(part_h);
     if (rc) return rc;
     rc = h->cfg.mode == EUP_MODE_PARITY ? parity_prepare_mask(h) : physics_prepare_mask(h);
     if (rc) return rc;

@@ -82,6 +82,7 @@ int fail(Handle *h, int code, const std::string &msg);
 size_t occupancy_lds_bytes(const Handle *h, int cap);
 bool stream_stores(const Handle *h, double bytes);
 int hip_check(Handle *h, hipError_t e, const char *what);
+int pinned_ready(Handle *h, int64_t bytes); // h->pinned holds at least `bytes`
 
 // parity mode (eup_parity.hip)
 int parity_prepare_mask(Handle *h);

@@ -522,14 +522,12 @@ __global__ __launch_bounds__(kBlock) void k_classify(const uint8_t *__restrict__
     link_all[(size_t)t * kTile + (threadIdx.x & 63)] = lm;
 }
 
-__global__ void k_uniform_links(uint32_t *__restrict__ link)
-{
-    link[threadIdx.x] = threadIdx.x < kTile ? 0u : 0x80000000u;
-}
-
+// the link masks of the mixed tiles, then those of a fluid and of a solid tile (two-step kernel)
 __global__ void k_compact_links(const int32_t *__restrict__ code, const uint32_t *__restrict__ link_all,
-                                uint32_t tiles, uint32_t *__restrict__ link)
+                                uint32_t tiles, uint32_t *__restrict__ link, int64_t mixed)
 {
+    if (blockIdx.x == 0 && threadIdx.x < 2 * kTile)
+        link[mixed * kTile + threadIdx.x] = threadIdx.x < kTile ? 0u : 0x80000000u;
     const uint32_t t = blockIdx.x * (kBlock / kTile) + (threadIdx.x >> 6);
     if (t >= tiles) return;
     const int32_t c = code[t];
@@ -1042,13 +1040,8 @@ int physics_prepare_mask(Handle *h)
             rc = EUP_EHIP;
     }
     if (!rc) {
-        // the masks of a fluid and of a solid tile after the mixed tiles' (two-step kernel)
-        hipLaunchKernelGGL(k_uniform_links, dim3(1), dim3(2 * kTile), 0, h->stream, h->link_mask + nm * kTile);
-        if (hip_check(h, hipGetLastError(), "uniform links")) rc = EUP_EHIP;
-    }
-    if (!rc && nm > 0) {
         hipLaunchKernelGGL(k_compact_links, dim3(grid), dim3(kBlock), 0, h->stream, h->tile_code,
-                           link_all, (uint32_t)g.tiles, h->link_mask);
+                           link_all, (uint32_t)g.tiles, h->link_mask, nm);
         if (hip_check(h, hipGetLastError(), "compact links")) rc = EUP_EHIP;
     }
     if (!rc && nm > 0) {
