@@ -111,7 +111,7 @@ static void release(Handle *h)
     if (h->stream) hipStreamSynchronize(h->stream);
     void *ptrs[] = {h->alloc[0], h->alloc[1], h->obs_stage, h->solid, h->solid_list,
                     h->tile_code, h->link_mask, h->mixed_list, h->outlet[0], h->outlet[1], h->diag,
-                    h->site19, h->grey, h->grey_zero, h->work};
+                    h->ticket, h->grey, h->grey_zero, h->work};
     for (void *p : ptrs)
         if (p) hipFree(p);
     if (h->pinned) hipHostFree(h->pinned);

@@ -7,6 +7,7 @@
 // them in the reference's loop order, so the host sums them exactly as flux_X/flux_Y do.  The
 // momentum-exchange force and the global means are wavefront-reduced on the GPU in a fixed order
 // (deterministic run to run).
+#include <algorithm>
 #include <mutex>
 #include <type_traits>
 #include <vector>
@@ -26,6 +27,8 @@ namespace eup {
 namespace {
 
 constexpr int kRedBlocks = 2048;
+constexpr int kTicketBlocks = 256; // largest grid whose last block adds the partial sums
+constexpr int64_t kResultBytes = 4096; // of pinned memory for a few results
 
 // population q of interior site (i, j, k) (1-based) as double
 struct ParityAcc {
@@ -148,8 +151,33 @@ __device__ __forceinline__ void block_reduce(double (&v)[NV], double *partial)
     }
 }
 
+// The blocks' partial sums and, with a ticket (0 between launches), by the block that ends last their
+// sum, into pinned host memory: thread b of that block adds the partials b, b + 256, ..., so the
+// order does not depend on which block it is, and is that of k_final.  One launch instead of two
+// and no copy of the result: a step, its drag and a probe on 48 x 24 x 16 take 54.6 us instead of 78.4.  Every ticket is a release to
+// the other XCDs, and 2048 of them cost more than the second launch: kTicketBlocks.
 template <int NV>
-__global__ void k_final(const double *partial, int nblocks, double *out)
+__device__ __forceinline__ void grid_reduce(double (&v)[NV], double *partial, uint32_t *ticket, double *out)
+{
+    __shared__ bool last;
+    block_reduce<NV>(v, partial);
+    if (!ticket) return;
+    if (threadIdx.x == 0)
+        last = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
+    __syncthreads();
+    if (!last) return;
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+#pragma unroll
+    for (int c = 0; c < NV; ++c) v[c] = 0.0;
+    for (uint32_t b = threadIdx.x; b < gridDim.x; b += kBlock)
+#pragma unroll
+        for (int c = 0; c < NV; ++c) v[c] += partial[(int64_t)b * NV + c];
+    block_reduce<NV>(v, out - (int64_t)blockIdx.x * NV);
+    if (threadIdx.x == 0) *ticket = 0;
+}
+
+template <int NV>
+__global__ __launch_bounds__(kBlock) void k_final(const double *partial, int nblocks, double *out)
 {
     double v[NV];
 #pragma unroll
@@ -163,7 +191,7 @@ __global__ void k_final(const double *partial, int nblocks, double *out)
 // momentum exchange over all interior sites (parity layout), neighbour test on the solid flags
 template <typename Acc>
 __global__ __launch_bounds__(kBlock) void k_mem_sites(Acc acc, const uint8_t *solid, int xopen,
-                                                      double *partial)
+                                                      double *partial, uint32_t *ticket, double *out)
 {
     const int l = acc.l, m = acc.m, n = acc.n;
     const int64_t N = (int64_t)l * m * n;
@@ -189,7 +217,7 @@ __global__ __launch_bounds__(kBlock) void k_mem_sites(Acc acc, const uint8_t *so
             v[2] += czs[p] * f2;
         }
     }
-    block_reduce<3>(v, partial);
+    grid_reduce<3>(v, partial, ticket, out);
 }
 
 // momentum exchange over the mixed tiles only (physics layout): bit opp(p) of the link mask of a
@@ -197,7 +225,7 @@ __global__ __launch_bounds__(kBlock) void k_mem_sites(Acc acc, const uint8_t *so
 template <typename S>
 __global__ __launch_bounds__(kBlock) void k_mem_tiles(PhysAcc<S> acc, const int32_t *mixed_list,
                                                       int64_t nmixed, const uint32_t *link, int tpr,
-                                                      double *partial)
+                                                      double *partial, uint32_t *ticket, double *out)
 {
     const int cxs[18] = {1, 1, 1, 1, 1, 0, 0, 0, 0, -1, -1, -1, -1, -1, 0, 0, 0, 0};
     const int cys[18] = {-1, 0, 1, 0, 0, 0, 1, 1, 1, -1, 0, 1, 0, 0, 0, -1, -1, -1};
@@ -214,15 +242,21 @@ __global__ __launch_bounds__(kBlock) void k_mem_tiles(PhysAcc<S> acc, const int3
         const int i = (int)(t - row * tpr) * kTile + lane;
         if (i >= acc.l) continue;
         const int j = (int)(row % acc.m), k = (int)(row / acc.m);
+        // all 18 loads at once (one behind a branch each waited for the one before: 170 x 77 x 51 with 3 %
+        // scattered solid sites, FP32, 25.5 us, now 12.1); a site without
+        // the link reads its population 0 and adds a zero, which changes no sum
+        S x[18];
+#pragma unroll
+        for (int p = 0; p < 18; ++p) x[p] = acc.base[acc.ix((lm >> opp[p]) & 1u ? p : 0, i, j, k)];
+#pragma unroll
         for (int p = 0; p < 18; ++p) {
-            if (!((lm >> opp[p]) & 1u)) continue;
-            const double f2 = 2.0 * acc(p, i + 1, j + 1, k + 1);
+            const double f2 = (lm >> opp[p]) & 1u ? 2.0 * Store<S>::load64(x[p], acc.ref.r[p], p) : 0.0;
             v[0] += cxs[p] * f2;
             v[1] += cys[p] * f2;
             v[2] += czs[p] * f2;
         }
     }
-    block_reduce<3>(v, partial);
+    grid_reduce<3>(v, partial, ticket, out);
 }
 
 // velocity of one site as the reference's binary VTK writers compute it (vtk_xy.binary.F90:93-115):
@@ -311,20 +345,21 @@ __global__ void k_vtk_vorticity(Acc acc, int k0, int64_t t0, int64_t count, floa
     out[o] = 0.5f * (mom[0] - mom[1]) - 0.5f * (mom[3] - mom[2]);
 }
 
-template <typename Acc>
+// I: unsigned type that holds the site numbers (divided twice per site; 32 bits where they suffice:
+// 192 x 768 x 768, e3m12, 1.63 -> 1.47 ms)
+template <typename Acc, typename I>
 __global__ __launch_bounds__(kBlock) void k_diagno(Acc acc, const uint8_t *solid, double *partial)
 {
-    const int l = acc.l, m = acc.m, n = acc.n;
-    const int64_t N = (int64_t)l * m * n;
+    const I l = (I)acc.l, m = (I)acc.m;
+    const I N = l * m * (I)acc.n;
     double v[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-    for (int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; s < N; s += (int64_t)gridDim.x * blockDim.x) {
+    for (I s = (I)blockIdx.x * kBlock + threadIdx.x; s < N; s += (I)gridDim.x * kBlock) {
         double rho, xj, yj, zj;
         if (solid[s]) {
             rho = 1.0; xj = 0.0; yj = 0.0; zj = 0.0;
         } else {
-            const int i = 1 + (int)(s % l);
-            const int64_t r = s / l;
-            const int j = 1 + (int)(r % m), k = 1 + (int)(r / m);
+            const I r = s / l, z = r / m;
+            const int i = 1 + (int)(s - r * l), j = 1 + (int)(r - z * m), k = 1 + (int)z;
             double x[19];
 #pragma unroll
             for (int q = 0; q < 19; ++q) x[q] = acc(q, i, j, k);
@@ -397,18 +432,15 @@ int ensure_diag(Handle *h, int64_t len)
 
 int diag_site(Handle *h, int i, int j, int k, double out[19])
 {
-    if (!h->site19 && hip_check(h, hipMalloc((void **)&h->site19, sizeof(double) * 32), "hipMalloc"))
-        return EUP_EHIP;
+    if (pinned_ready(h, kResultBytes)) return EUP_EHIP;
+    double *res = reinterpret_cast<double *>(h->pinned);
     int rc = with_acc(h, [&](auto acc) {
-        hipLaunchKernelGGL((k_site19<decltype(acc)>), dim3(1), dim3(64), 0, h->stream, acc, i, j, k,
-                           h->site19);
+        hipLaunchKernelGGL((k_site19<decltype(acc)>), dim3(1), dim3(64), 0, h->stream, acc, i, j, k, res);
         return hip_check(h, hipGetLastError(), "site gather") ? EUP_EHIP : 0;
     });
     if (rc) return rc;
-    if (hip_check(h, hipMemcpyAsync(out, h->site19, sizeof(double) * 19, hipMemcpyDeviceToHost, h->stream),
-                  "copy site") ||
-        hip_check(h, hipStreamSynchronize(h->stream), "sync"))
-        return EUP_EHIP;
+    if (hip_check(h, hipStreamSynchronize(h->stream), "sync")) return EUP_EHIP;
+    memcpy(out, res, sizeof(double) * 19);
     return 0;
 }
 
@@ -545,38 +577,49 @@ int diag_drag_cv_noalloc(Handle *h, const int32_t box[6], double *fx, double *fy
     return drag_axis(h, box, 1, fy, s, kNoAllocFace);
 }
 
+// the scratch of a reduction to nv values: partial sums, ticket and result
+static int reduce_ready(Handle *h, int nv)
+{
+    if (ensure_diag(h, nv * kRedBlocks) || pinned_ready(h, kResultBytes)) return EUP_EHIP;
+    if (h->ticket) return 0;
+    if (hip_check(h, hipMalloc((void **)&h->ticket, sizeof(uint32_t)), "hipMalloc ticket") ||
+        hip_check(h, hipMemsetAsync(h->ticket, 0, sizeof(uint32_t), h->stream), "clear ticket"))
+        return EUP_EHIP;
+    return 0;
+}
+
 int diag_drag_mem(Handle *h, double F[3])
 {
-    int rc = ensure_diag(h, 3 * kRedBlocks + 8);
-    if (rc) return rc;
     const int xopen = h->cfg.front != EUP_FACE_PERIODIC;
-    if (h->cfg.mode == EUP_MODE_PARITY) {
-        hipLaunchKernelGGL((k_mem_sites<ParityAcc>), dim3(kRedBlocks), dim3(kBlock), 0, h->stream,
-                           parity_acc(h), h->solid, xopen, h->diag);
-    } else if (h->tiles_mixed > 0) {
-        rc = with_acc(h, [&](auto acc) -> int {
-            using A = decltype(acc);
-            if constexpr (std::is_same_v<A, ParityAcc>) {
-                return 0;
-            } else {
-                using S = typename A::value_type;
-                hipLaunchKernelGGL((k_mem_tiles<S>), dim3(kRedBlocks), dim3(kBlock), 0, h->stream, acc,
-                                   h->mixed_list, h->tiles_mixed, h->link_mask, h->g.tiles_per_row,
-                                   h->diag);
-                return 0;
-            }
-        });
-        if (rc) return rc;
-    } else {
+    if (h->cfg.mode != EUP_MODE_PARITY && h->tiles_mixed == 0) {
         F[0] = F[1] = F[2] = 0.0;
         return 0;
     }
-    double *res = h->diag + 3 * kRedBlocks;
-    hipLaunchKernelGGL((k_final<3>), dim3(1), dim3(kBlock), 0, h->stream, h->diag, kRedBlocks, res);
-    if (hip_check(h, hipGetLastError(), "mem drag") ||
-        hip_check(h, hipMemcpyAsync(F, res, sizeof(double) * 3, hipMemcpyDeviceToHost, h->stream), "copy") ||
-        hip_check(h, hipStreamSynchronize(h->stream), "sync"))
+    int rc = reduce_ready(h, 3);
+    if (rc) return rc;
+    double *res = reinterpret_cast<double *>(h->pinned);
+    // physics: no more blocks than tiles to give them (the partials left out were zeros)
+    int blocks = kRedBlocks;
+    if (h->cfg.mode != EUP_MODE_PARITY)
+        blocks = (int)std::min<int64_t>(blocks, (h->tiles_mixed + kBlock / 64 - 1) / (kBlock / 64));
+    uint32_t *ticket = blocks <= kTicketBlocks ? h->ticket : nullptr;
+    rc = with_acc(h, [&](auto acc) -> int {
+        using A = decltype(acc);
+        if constexpr (std::is_same_v<A, ParityAcc>) {
+            hipLaunchKernelGGL((k_mem_sites<A>), dim3(blocks), dim3(kBlock), 0, h->stream, acc, h->solid, xopen,
+                               h->diag, ticket, res);
+        } else {
+            using S = typename A::value_type;
+            hipLaunchKernelGGL((k_mem_tiles<S>), dim3(blocks), dim3(kBlock), 0, h->stream, acc, h->mixed_list,
+                               h->tiles_mixed, h->link_mask, h->g.tiles_per_row, h->diag, ticket, res);
+        }
+        return 0;
+    });
+    if (rc) return rc;
+    if (!ticket) hipLaunchKernelGGL((k_final<3>), dim3(1), dim3(kBlock), 0, h->stream, h->diag, blocks, res);
+    if (hip_check(h, hipGetLastError(), "mem drag") || hip_check(h, hipStreamSynchronize(h->stream), "sync"))
         return EUP_EHIP;
+    for (int c = 0; c < 3; ++c) F[c] = res[c];
     return 0;
 }
 
@@ -608,20 +651,23 @@ int diag_vtk_vorticity(Handle *h, int k0, float *out)
 
 int diag_diagno(Handle *h, double out[5])
 {
-    int rc = ensure_diag(h, 5 * kRedBlocks + 8);
+    int rc = reduce_ready(h, 5);
     if (rc) return rc;
+    double *tot = reinterpret_cast<double *>(h->pinned);
     rc = with_acc(h, [&](auto acc) {
-        hipLaunchKernelGGL((k_diagno<decltype(acc)>), dim3(kRedBlocks), dim3(kBlock), 0, h->stream, acc,
-                           h->solid, h->diag);
+        using A = decltype(acc);
+        // (the last stride may pass the last site: it has to fit as well)
+        if (h->g.sites < INT32_MAX)
+            hipLaunchKernelGGL((k_diagno<A, uint32_t>), dim3(kRedBlocks), dim3(kBlock), 0, h->stream, acc, h->solid,
+                               h->diag);
+        else
+            hipLaunchKernelGGL((k_diagno<A, uint64_t>), dim3(kRedBlocks), dim3(kBlock), 0, h->stream, acc, h->solid,
+                               h->diag);
         return 0;
     });
     if (rc) return rc;
-    double *res = h->diag + 5 * kRedBlocks;
-    hipLaunchKernelGGL((k_final<5>), dim3(1), dim3(kBlock), 0, h->stream, h->diag, kRedBlocks, res);
-    double tot[5];
-    if (hip_check(h, hipGetLastError(), "diagno") ||
-        hip_check(h, hipMemcpyAsync(tot, res, sizeof(double) * 5, hipMemcpyDeviceToHost, h->stream), "copy") ||
-        hip_check(h, hipStreamSynchronize(h->stream), "sync"))
+    hipLaunchKernelGGL((k_final<5>), dim3(1), dim3(kBlock), 0, h->stream, h->diag, kRedBlocks, tot);
+    if (hip_check(h, hipGetLastError(), "diagno") || hip_check(h, hipStreamSynchronize(h->stream), "sync"))
         return EUP_EHIP;
     const double rdv = 1. / ((double)h->g.l * (double)h->g.m * (double)h->g.n);
     for (int c = 0; c < 5; ++c) out[c] = tot[c] * rdv;

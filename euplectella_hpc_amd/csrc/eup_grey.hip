@@ -453,7 +453,7 @@ template <typename R, bool BIG> __global__ __launch_bounds__(256) void k_adj_str
 // site takes the two halves' terms in the same order as the split kernels, so the result is
 // bit-identical to running k_adj_stream(t) and k_adj_collide(t - 1).  Bound by latency at two (FP32, 251
 // registers) and one (FP64) wavefronts per SIMD with every load of a half in flight: held to three
-// wavefronts, or with the loads in groups of 6, it spills or waits more (FP32 45 us; 65-90 us at
+// wavefronts, or with the loads in groups of 6, it spills or waits more (FP32 45 us; about 85 us at
 // three).
 template <typename R, bool BIG> __global__ __launch_bounds__(256) void k_adj_fused(AdjArgs<R> sa, AdjArgs<R> ca)
 {

@@ -65,7 +65,7 @@ struct Handle {
     // diagnostics scratch
     double *diag = nullptr;       // device scratch for reductions
     int64_t diag_len = 0;
-    double *site19 = nullptr;     // one site's 19 populations in FP64
+    uint32_t *ticket = nullptr;   // blocks of a reduction that have ended
     // grey mode
     void *grey = nullptr;         // solid fraction (compute type), l*m*n
     uint8_t *grey_zero = nullptr; // per 64 sites: no solid fraction there or next to them
