@@ -9,7 +9,9 @@ is measured for each storage in the same run (``accuracy``; ``qualified_16bit`` 
 storage that meets it at the workload's own tau, with its speed-up over FP32), beside the floor of
 each window: FP64 against FP64 started from its own state rounded once to FP32.
 
-A step is one fused collide+stream launch over the whole lattice.  MLUPS follows the reference's
+A step is one fused collide+stream pass over the whole lattice; FP32 and FP64 storage take two steps
+per launch, the state between them kept on the chip, so that their HBM bytes per step lie below the
+algorithmic bytes of single steps and the fraction of peak can pass 1.  MLUPS follows the reference's
 definition (all l*m*n sites per second, CODE/SRC/finalize.F90:107-108).  The roofline figure uses
 the algorithmic HBM bytes of the fluid sites actually updated (19 loads + 19 stores of the storage
 type each; solid sites are neither loaded nor stored), divided by the kernel time measured with HIP
@@ -17,7 +19,7 @@ events on the library's stream.
 
 Beside the nominal 8 TB/s peak the line carries the HBM rates the same GPU reaches in plain
 streams (eup_membw: copy / read / write of 2 GiB, one 16-byte vector per lane), and
-``roofline.traffic``, the HBM bytes per launch of the fused kernel that rocprofv3's FETCH_SIZE and
+``roofline.traffic``, the HBM bytes per step that rocprofv3's FETCH_SIZE and
 WRITE_SIZE counters gave for this workload and storage (calibrated on the copy stream; the summary
 is read from profiles/, null when no profile of this configuration is committed).
 
@@ -165,8 +167,9 @@ def hbm_streams(mib=2048, reps=10):
 
 
 def profiled_traffic(workload, storage):
-    """HBM bytes per fused-kernel launch from the committed rocprofv3 counter summary, or None."""
-    path = os.path.join(ROOT, "profiles", f"k_fused_{workload}_hbm_counters.txt")
+    """HBM bytes per step from the committed rocprofv3 counter summary, or None."""
+    kernel = "k_pair" if storage in ("f32", "f64") else "k_fused"
+    path = os.path.join(ROOT, "profiles", f"{kernel}_{workload}_hbm_counters.txt")
     if not os.path.exists(path):
         return None, None
     pat = re.compile(r"^traffic storage=(\S+) .*\bbytes=(\d+)")
@@ -662,8 +665,8 @@ def main(argv=None):
                      "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(prim["frac"], 4),
                      "traffic": traffic, "traffic_source": traffic_src,
                      "algorithmic_bytes": int(prim["fluid_sites"] * prim["bytes_per_site"]),
-                     "kernel": "k_fused" if args.mode == "physics" else
-                     "k_bb_gather + k_bb_scatter + k_ghost + k_stream_collide",
+                     "kernel": "k_bounce + k_ghost + k_stream_collide" if args.mode != "physics" else
+                     "k_pair (two steps per launch)" if args.storage in ("f32", "f64") else "k_fused",
                      "kernel_ms": round(prim["kernel_ms"], 4),
                      "bytes_per_site": prim["bytes_per_site"],
                      "hbm_streams_gbs": streams,
