@@ -11,7 +11,8 @@ each window: FP64 against FP64 started from its own state rounded once to FP32.
 
 A step is one fused collide+stream pass over the whole lattice; FP32 and FP64 storage take two steps
 per launch, the state between them kept on the chip, so that their HBM bytes per step lie below the
-algorithmic bytes of single steps and the fraction of peak can pass 1.  MLUPS follows the reference's
+algorithmic bytes of single steps and ``frac`` can pass 1; ``traffic_frac`` is the fraction of peak of
+the bytes they do move.  MLUPS follows the reference's
 definition (all l*m*n sites per second, CODE/SRC/finalize.F90:107-108).  The roofline figure uses
 the algorithmic HBM bytes of the fluid sites actually updated (19 loads + 19 stores of the storage
 type each; solid sites are neither loaded nor stored), divided by the kernel time measured with HIP
@@ -664,6 +665,8 @@ def main(argv=None):
         "roofline": {"bound": "hbm", "achieved": round(prim["achieved_gbs"], 1),
                      "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(prim["frac"], 4),
                      "traffic": traffic, "traffic_source": traffic_src,
+                     "traffic_frac": (round(traffic / (prim["kernel_ms"] * 1e6) / HBM_PEAK_GBS, 4)
+                                      if traffic else None),
                      "algorithmic_bytes": int(prim["fluid_sites"] * prim["bytes_per_site"]),
                      "kernel": "k_bounce + k_ghost + k_stream_collide" if args.mode != "physics" else
                      "k_pair (two steps per launch)" if args.storage in ("f32", "f64") else "k_fused",
