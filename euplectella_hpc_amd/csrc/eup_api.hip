@@ -449,6 +449,7 @@ static int set_pops(eup_handle *h, int q, int nq, const double *a)
     int rc = h->cfg.mode == EUP_MODE_PARITY ? parity_set_pops(h, q, nq, a) : physics_set_pops(h, q, nq, a);
     if (rc) return rc;
     h->pops_set |= ((1u << nq) - 1) << q;
+    if (nq == 19) h->stepped = false;
     return 0;
 }
 

@@ -57,6 +57,7 @@ struct Handle {
     int64_t tiles_fluid = 0, tiles_mixed = 0, tiles_solid = 0;
     int32_t *mixed_list = nullptr; // tile indices of mixed tiles
     void *outlet[2] = {nullptr, nullptr}; // outlet ghost plane, 5 x m x n (compute type)
+    bool stepped = false;          // physics mode: the two buffers may differ at sites that a step wrote
     bool outlet_dirty = true;      // the host wrote populations: physics and grey mode recompute the
                                    // outlet plane, parity mode refills the constant inflow plane
     size_t fused_lds = (size_t)-1; // dynamic LDS per block of the fused kernel (occupancy cap)

@@ -535,6 +535,22 @@ __global__ void k_compact_links(const int32_t *__restrict__ code, const uint32_t
     link[(size_t)c * kTile + (threadIdx.x & 63)] = link_all[(size_t)t * kTile + (threadIdx.x & 63)];
 }
 
+// The populations of the solid sites (link_all, bit 31) from the current buffer into the other one: no
+// step writes them, so a site that a mask set between steps makes solid would show its last value and
+// the one before by turns.
+template <typename S>
+__global__ __launch_bounds__(kBlock) void k_freeze(const S *__restrict__ cur, S *__restrict__ other,
+                                                   const uint32_t *__restrict__ link_all, uint32_t tiles)
+{
+    const uint32_t t = blockIdx.x * (kBlock / kTile) + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (t >= tiles || !(link_all[(size_t)t * kTile + lane] & 0x80000000u)) return;
+#pragma unroll
+    for (int q = 0; q < 19; ++q) {
+        const size_t e = (size_t)t * kTileElems + q * kTile + lane;
+        other[e] = cur[e];
+    }
+}
+
 // ---------------------------------------------------------------------------------------------
 // state conversion and outlet refresh
 // ---------------------------------------------------------------------------------------------
@@ -940,6 +956,7 @@ int physics_steps(Handle *h, int nsteps)
         int rc = physics_refresh_outlet(h);
         if (rc) return rc;
     }
+    h->stepped = h->stepped || nsteps > 0;
     return dispatch(h, [&](auto *p) -> int {
         using S = std::remove_pointer_t<decltype(p)>;
         int t = 0, rc = 0;
@@ -991,6 +1008,7 @@ int init_equilibrium(Handle *h, double ux, double uy, double uz, double noise, u
         if (rc) return rc;
     }
     h->outlet_dirty = true;
+    h->stepped = false;
     return hip_check(h, hipStreamSynchronize(h->stream), "sync") ? EUP_EHIP : 0;
 }
 
@@ -1010,6 +1028,14 @@ int physics_prepare_mask(Handle *h)
     hipLaunchKernelGGL(k_classify, dim3(grid), dim3(kBlock), 0, h->stream, h->solid, g.l, g.m, g.n,
                        g.tiles_per_row, (uint32_t)g.tiles, (int)x_open(h), (int)noskip, cls, link_all);
     if (hip_check(h, hipGetLastError(), "classify")) rc = EUP_EHIP;
+    if (!rc && h->stepped)
+        rc = dispatch(h, [&](auto *p) {
+            using S = std::remove_pointer_t<decltype(p)>;
+            hipLaunchKernelGGL((k_freeze<S>), dim3(grid), dim3(kBlock), 0, h->stream,
+                               static_cast<const S *>(h->buf[h->cur]), static_cast<S *>(h->buf[h->cur ^ 1]), link_all,
+                               (uint32_t)g.tiles);
+            return hip_check(h, hipGetLastError(), "freeze") ? EUP_EHIP : 0;
+        });
     uint8_t *cls_h = nullptr;
     int32_t *code_h = nullptr;
     if (!rc && (hip_check(h, hipHostMalloc((void **)&cls_h, g.tiles), "hipHostMalloc") ||

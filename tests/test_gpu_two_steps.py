@@ -55,3 +55,39 @@ def test_chunks_of_planes(chunk, storage, monkeypatch):
     two = after(shape, storage, True, mask, 4, "1", monkeypatch)
     for a, b in zip(one, two):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("storage", ["f32", "f64", "f16", "bf16", "e3m12"])
+@pytest.mark.parametrize("x_open", [True, False])
+@pytest.mark.parametrize("shape", [(70, 14, 9), (128, 6, 5)])
+def test_mask_changed_between_steps(shape, x_open, storage, monkeypatch):
+    """A site that a new mask makes solid keeps, from the commit on, the values it had there, whatever
+    the number of steps that follow and however they are taken; released again, it flows on from them."""
+    from euplectella_hpc_amd.lib import Lattice
+
+    print(f"mask changed {shape} x_open={x_open} {storage}", flush=True)
+    masks = [geometry.scattered(*shape, fraction=f, seed=s).astype(bool) for f, s in ((0.05, 5), (0.1, 6), (0.05, 7))]
+    masks[1][:, : shape[1] // 2, :64] = True  # whole tiles of solid sites
+    for steps in (1, 2, 5):
+        runs = []
+        for pair in ("0", "1"):
+            monkeypatch.setenv("EUP_PAIR", pair)
+            with Lattice(*shape, svisc=0.05, u_inflow=0.05, mode="physics", storage=storage, x_open=x_open,
+                         fgrad=0.0 if x_open else 1e-5) as lat:
+                lat.set_mask(masks[0])
+                lat.init_equilibrium(0.05, 0.01, -0.02, 1e-2, 3)
+                lat.step(3)
+                before = lat.get_state()
+                lat.set_mask(masks[1])
+                lat.step(steps)
+                after = lat.get_state()
+                lat.set_mask(masks[2])
+                lat.step(2)
+                runs.append((after, lat.get_state(), lat.drag_mem()))
+            solid = masks[1]
+            inner = np.s_[:, 1:-1, 1:-1, 1:-1]
+            assert np.array_equal(after[inner][:, solid], before[inner][:, solid])
+            assert not np.array_equal(after[inner][:, ~solid], before[inner][:, ~solid])
+        for a, b in zip(*runs):
+            assert np.isfinite(a).all()
+            assert np.array_equal(a, b)
