@@ -9,9 +9,9 @@ is measured for each storage in the same run (``accuracy``; ``qualified_16bit`` 
 storage that meets it at the workload's own tau, with its speed-up over FP32), beside the floor of
 each window: FP64 against FP64 started from its own state rounded once to FP32.
 
-A step is one fused collide+stream pass over the whole lattice; FP32 and FP64 storage take two steps
-per launch, the state between them kept on the chip, so that their HBM bytes per step lie below the
-algorithmic bytes of single steps and ``frac`` can pass 1; ``traffic_frac`` is the fraction of peak of
+A step is one fused collide+stream pass over the whole lattice; where FP32 and FP64 storage take two
+steps per launch (the library says so: eup_steps_per_launch), the state between them kept on the chip,
+their HBM bytes per step lie below the algorithmic bytes of single steps and ``frac`` can pass 1; ``traffic_frac`` is the fraction of peak of
 the bytes they do move.  MLUPS follows the reference's
 definition (all l*m*n sites per second, CODE/SRC/finalize.F90:107-108).  The roofline figure uses
 the algorithmic HBM bytes of the fluid sites actually updated (19 loads + 19 stores of the storage
@@ -143,6 +143,7 @@ def run_one(wl, storage, mask, steps, warmup, chain=True, mode="physics"):
         kernel_s = gpu_ms / 1e3 / steps
         bps = 2 * 19 * storage_bytes(storage)
         achieved = fluid * bps / kernel_s / 1e9
+        per_launch = lat.steps_per_launch(steps)
         probe = lat.probe(wl["l"] * 8 // 20, wl["m"] * 9 // 16, wl["n"] // 2 - 5)
         return {
             "finite": bool(np.all(np.isfinite(probe))),
@@ -154,6 +155,7 @@ def run_one(wl, storage, mask, steps, warmup, chain=True, mode="physics"):
             "achieved_gbs": achieved,
             "frac": achieved / HBM_PEAK_GBS,
             "fluid_sites": fluid,
+            "steps_per_launch": per_launch,
             "tiles": {k: info[k] for k in ("tiles", "tiles_fluid", "tiles_mixed", "tiles_solid")},
         }
     finally:
@@ -167,9 +169,12 @@ def hbm_streams(mib=2048, reps=10):
     return {k: round(float(v), 1) for k, v in r.items()}
 
 
-def profiled_traffic(workload, storage):
-    """HBM bytes per step from the committed rocprofv3 counter summary, or None."""
-    kernel = "k_pair" if storage in ("f32", "f64") else "k_fused"
+def step_kernel(steps_per_launch):
+    return "k_pair" if steps_per_launch == 2 else "k_fused"
+
+
+def profiled_traffic(workload, storage, kernel):
+    """HBM bytes per step of the kernel that ran, from the committed rocprofv3 counter summary, or None."""
     path = os.path.join(ROOT, "profiles", f"{kernel}_{workload}_hbm_counters.txt")
     if not os.path.exists(path):
         return None, None
@@ -637,7 +642,8 @@ def main(argv=None):
         print(f"[bench] {st}: {also[st]['mlups']:.0f} MLUPS, kernel {also[st]['kernel_ms']:.3f} ms",
               file=sys.stderr, flush=True)
     streams = None if args.no_streams else hbm_streams()
-    traffic, traffic_src = (profiled_traffic(args.workload, args.storage) if args.mode == "physics"
+    traffic, traffic_src = (profiled_traffic(args.workload, args.storage, step_kernel(prim["steps_per_launch"]))
+                            if args.mode == "physics"
                             else (None, None))
     cpu = None if args.no_cpu else cpu_baseline(wl, mask=mask)
     out = {
@@ -669,7 +675,8 @@ def main(argv=None):
                                       if traffic else None),
                      "algorithmic_bytes": int(prim["fluid_sites"] * prim["bytes_per_site"]),
                      "kernel": "k_bounce + k_ghost + k_stream_collide" if args.mode != "physics" else
-                     "k_pair (two steps per launch)" if args.storage in ("f32", "f64") else "k_fused",
+                     step_kernel(prim["steps_per_launch"]) +
+                     (" (two steps per launch)" if prim["steps_per_launch"] == 2 else ""),
                      "kernel_ms": round(prim["kernel_ms"], 4),
                      "bytes_per_site": prim["bytes_per_site"],
                      "hbm_streams_gbs": streams,

@@ -744,6 +744,12 @@ int eup_get_info(eup_handle *h, eup_info *info)
     return 0;
 }
 
+int eup_steps_per_launch(eup_handle *h, int32_t nsteps)
+{
+    if (!h || nsteps < 1) return fail(h, EUP_EINVAL, "eup_steps_per_launch: null handle or nsteps < 1");
+    return h->cfg.mode == EUP_MODE_PHYSICS ? physics_steps_per_launch(h, nsteps) : 1;
+}
+
 void *eup_stream(eup_handle *h) { return h ? (void *)h->stream : nullptr; }
 
 } // extern "C"

@@ -92,6 +92,7 @@ int parity_step(Handle *h);
 // physics mode (eup_physics.hip)
 int physics_prepare_mask(Handle *h);
 int physics_steps(Handle *h, int nsteps);
+int physics_steps_per_launch(Handle *h, int nsteps);
 int physics_refresh_outlet(Handle *h);
 // nq populations from q (0-based) on between the reference's ghosted FP64 arrays and the state
 int physics_set_pops(Handle *h, int q, int nq, const double *a); // -> both buffers

@@ -950,6 +950,15 @@ template <typename F> int dispatch(Handle *h, F &&f)
 
 } // namespace
 
+int physics_steps_per_launch(Handle *h, int nsteps)
+{
+    return dispatch(h, [&](auto *p) {
+        using S = std::remove_pointer_t<decltype(p)>;
+        if constexpr (kPairs<S>) return nsteps > 1 && pair_better<S>(h) ? 2 : 1;
+        else return 1;
+    });
+}
+
 int physics_steps(Handle *h, int nsteps)
 {
     if (nsteps > 0 && h->outlet_dirty) {
@@ -961,7 +970,7 @@ int physics_steps(Handle *h, int nsteps)
         using S = std::remove_pointer_t<decltype(p)>;
         int t = 0, rc = 0;
         if constexpr (kPairs<S>) {
-            if (nsteps > 1 && pair_better<S>(h)) {
+            if (physics_steps_per_launch(h, nsteps) == 2) {
                 auto launches = [&](auto nt) {
                     constexpr bool NT = decltype(nt)::value;
                     return x_open(h) ? pair_launches<S, true, NT>(h, nsteps / 2) : pair_launches<S, false, NT>(h, nsteps / 2);

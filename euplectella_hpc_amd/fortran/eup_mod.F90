@@ -185,6 +185,12 @@ module eup
          type(eup_info), intent(out) :: info
       end function eup_get_info
 
+      integer(c_int) function eup_steps_per_launch(h, nsteps) bind(c, name='eup_steps_per_launch')
+         import :: c_int, c_int32_t, c_ptr
+         type(c_ptr), value :: h
+         integer(c_int32_t), value :: nsteps
+      end function eup_steps_per_launch
+
       type(c_ptr) function eup_stream(h) bind(c, name='eup_stream')
          import :: c_ptr
          type(c_ptr), value :: h

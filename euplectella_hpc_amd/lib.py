@@ -33,7 +33,7 @@ FLAG_SHIFTED_DEVIATION = 2
 EXPORTS = ("eup_create", "eup_destroy", "eup_last_error", "eup_set_mask", "eup_set_pops",
            "eup_get_pops", "eup_set_state", "eup_get_state", "eup_step", "eup_step_timed",
            "eup_sync", "eup_drag_cv", "eup_drag_mem", "eup_probe", "eup_diagno", "eup_vtk_velocity",
-           "eup_vtk_vorticity", "eup_get_info",
+           "eup_vtk_vorticity", "eup_get_info", "eup_steps_per_launch",
            "eup_stream", "eup_abi_version", "eup_set_grey", "eup_set_grey_device",
            "eup_grey_force", "eup_grey_objective", "eup_grey_objective_device", "eup_membw",
            "eup_init_equilibrium", "eup_set_omega", "eup_add_obstacles", "eup_commit_obstacles",
@@ -110,6 +110,7 @@ def load():
     L.eup_vtk_velocity.argtypes = [vp, i32, i32, fp]
     L.eup_vtk_vorticity.argtypes = [vp, i32, fp]
     L.eup_get_info.argtypes = [vp, ctypes.POINTER(EupInfo)]
+    L.eup_steps_per_launch.argtypes = [vp, i32]
     L.eup_stream.argtypes = [vp]
     L.eup_stream.restype = vp
     L.eup_abi_version.argtypes = []
@@ -406,6 +407,13 @@ class Lattice:
         self._check(self.L.eup_get_info(self.h, ctypes.byref(inf)))
         return {k: (list(getattr(inf, k)) if k == "bbox" else getattr(inf, k))
                 for k, _ in EupInfo._fields_}
+
+    def steps_per_launch(self, nsteps=2):
+        """Time steps per kernel launch (2 or 1) in a call of ``nsteps`` with the present mask."""
+        rc = self.L.eup_steps_per_launch(self.h, int(nsteps))
+        if rc < 0:
+            self._check(rc)
+        return rc
 
     def stream(self):
         return self.L.eup_stream(self.h)

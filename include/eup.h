@@ -241,6 +241,11 @@ int eup_grey_objective_device(eup_handle *h, int32_t t0, int32_t t1, int32_t eve
 
 int eup_get_info(eup_handle *h, eup_info *info);
 
+/* Time steps per kernel launch in a call of nsteps (>= 1) steps with the present mask: 2 where
+ * physics mode takes them in pairs (an odd last step on its own), 1 otherwise.  The state is the same
+ * either way, bit for bit; a caller that reports kernel times or traffic needs to know which ran. */
+int eup_steps_per_launch(eup_handle *h, int32_t nsteps);
+
 /* The handle's HIP stream (hipStream_t) as an opaque pointer, for callers that order their own
  * work (timing events, PyTorch) with the library's. */
 void *eup_stream(eup_handle *h);

@@ -48,3 +48,15 @@ def test_seed_distribution_counts_and_orders():
     assert d["f16"] == {"runs": 4, "met": 2, "min": 5e-4, "median": 1.5e-3, "max": 8e-3}
     assert d["f32"]["met"] == 4 and d["f32"]["runs"] == 4
     assert bench.FLOOR not in d  # no window held it
+
+
+def test_traffic_is_that_of_the_kernel_that_ran():
+    sys.path.insert(0, ROOT)
+    import bench
+
+    two, src2 = bench.profiled_traffic("sponge_512x256x256", "f32", bench.step_kernel(2))
+    one, src1 = bench.profiled_traffic("sponge_512x256x256", "f32", bench.step_kernel(1))
+    assert src2.endswith("k_pair_sponge_512x256x256_hbm_counters.txt")
+    assert src1.endswith("k_fused_sponge_512x256x256_hbm_counters.txt")
+    assert two < 0.6 * one
+    assert bench.profiled_traffic("cylinder_128x64x64", "f32", bench.step_kernel(2)) == (None, None)

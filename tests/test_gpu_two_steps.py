@@ -91,3 +91,17 @@ def test_mask_changed_between_steps(shape, x_open, storage, monkeypatch):
         for a, b in zip(*runs):
             assert np.isfinite(a).all()
             assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("mode,storage,pairs", [("physics", "f32", 2), ("physics", "f64", 2), ("physics", "f16", 1),
+                                                ("physics", "e3m12", 1), ("parity", "f64", 1), ("grey", "f32", 1)])
+def test_steps_per_launch_says_which_form_runs(mode, storage, pairs, monkeypatch):
+    from euplectella_hpc_amd.lib import EupError, Lattice
+
+    with Lattice(64, 12, 7, svisc=0.05, u_inflow=0.05, mode=mode, storage=storage) as lat:
+        monkeypatch.setenv("EUP_PAIR", "1")
+        assert [lat.steps_per_launch(n) for n in (1, 2, 3)] == [1, pairs, pairs]
+        monkeypatch.setenv("EUP_PAIR", "0")
+        assert lat.steps_per_launch(2) == 1
+        with pytest.raises(EupError):
+            lat.steps_per_launch(0)
