@@ -870,13 +870,18 @@ template <typename S> PairMap pair_map(const Handle *h, double *us)
     return pm;
 }
 
-// Whether the handle's steps are taken two per launch: where a pair is expected to be at least a tenth
-// faster than two single steps (columns with obstacles cost a pair up to that much more), these at the
-// 6.1 TB/s and 2.5 us per launch that they reach (0.5 us with cached stores).  Measured, single
-// against pair per step, without obstacles: FP32 64 x 64 x 64 8.5 / 10.1 us (single), 128 x 64 x 64
-// 14.1 / 14.7 (single), 170 x 77 x 51 20.0 / 18.7, 256 x 128 x 128 105 / 82, 680 x 340 x 4 27.3 / 30.8 (single),
-// 512 x 256 x 256 813 / 571; FP64 128 x 64 x 64 25.7 / 28.8 (single), 256 x 128 x 128 210 / 178,
-// 512 x 256 x 256 1659 / 1285.
+// Whether the handle's steps are taken two per launch: where a pair is expected to be faster than two
+// single steps by more than the estimates' error, these at the 6.1 TB/s and 2.5 us per launch that they
+// reach (0.5 us with cached stores).  All-solid tiles cost a single step nothing and a pair all but its
+// stores (a tenth); their price of 1/2 here and the margin of 1.075 are those that lost least against
+// the faster form over 3216 lattices of 60 000 to 12 million sites with walls, grains, scattered sites
+// and bodies (0.9 % on average; 4.5 % with solid tiles priced like others, which took pairs up to 2.7
+// times slower).  Tiles with obstacles cost both forms alike, and the padding of a row's last tile does
+// cost a single step what a full tile does.  Measured, single against pair per step, without obstacles:
+// FP32 64 x 64 x 64 8.5 / 10.1 us (single), 128 x 64 x 64 14.1 / 14.7 (single), 170 x 77 x 51 20.0 / 18.7,
+// 256 x 128 x 128 105 / 82, 680 x 340 x 4 27.3 / 30.8 (single), 65 x 256 x 256 210 / 118, 512 x 256 x 256
+// 807 / 569, with 25, 40 and 60 % of all-solid tiles 625 / 559, 529 / 548 and 363 / 532; FP64 128 x 64 x
+// 64 25.7 / 28.8 (single), 256 x 128 x 128 210 / 178, 512 x 256 x 256 1659 / 1285.
 template <typename S> bool pair_better(const Handle *h)
 {
     const Geometry &g = h->g;
@@ -886,7 +891,8 @@ template <typename S> bool pair_better(const Handle *h)
     if (const char *e = getenv("EUP_PAIR")) return atoi(e) != 0;
     double us;
     pair_map<S>(h, &us);
-    return 1.1 * us < 2.0 * ((stream_stores(h, two_states<S>(h)) ? 2.5 : 0.5) + two_states<S>(h) / 6.1e6);
+    const double bytes = two_states<S>(h), solid = (double)h->tiles_solid / (double)g.tiles;
+    return 1.075 * us * (1.0 - 0.5 * solid) < 2.0 * ((stream_stores(h, bytes) ? 2.5 : 0.5) + bytes * (1.0 - solid) / 6.1e6);
 }
 
 template <typename S, bool XOPEN, bool NT> int pair_launches(Handle *h, int count)

@@ -105,3 +105,21 @@ def test_steps_per_launch_says_which_form_runs(mode, storage, pairs, monkeypatch
         assert lat.steps_per_launch(2) == 1
         with pytest.raises(EupError):
             lat.steps_per_launch(0)
+
+
+@pytest.mark.parametrize("storage", ["f32", "f64"])
+def test_mostly_solid_lattices_take_single_steps(storage):
+    """A single step skips tiles that are solid throughout, a pair does not: the default follows the mask."""
+    from euplectella_hpc_amd.lib import Lattice
+
+    l, m, n = 192, 96, 96
+    mask = np.zeros((n, m, l), bool)
+    with Lattice(l, m, n, svisc=0.05, u_inflow=0.05, mode="physics", storage=storage) as lat:
+        lat.set_mask(mask)
+        assert lat.steps_per_launch(2) == 2
+        mask[:, : 7 * m // 10] = True
+        lat.set_mask(mask)
+        assert lat.steps_per_launch(2) == 1
+        mask[:, 1:] = False
+        lat.set_mask(mask)
+        assert lat.steps_per_launch(2) == 2
