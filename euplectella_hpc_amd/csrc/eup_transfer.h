@@ -11,7 +11,6 @@
 #include <string.h>
 
 #include <atomic>
-#include <system_error>
 #include <thread>
 
 #include "eup_internal.h"
@@ -76,7 +75,7 @@ int transfer(Handle *h, char *host, int64_t bytes, int64_t unit, F &&launch)
                     while (workers.load(std::memory_order_acquire) == 0) std::this_thread::yield();
                     work(w, workers.load(std::memory_order_acquire));
                 });
-        } catch (const std::system_error &) { // no more threads to be had: those that run do the work
+        } catch (...) { // no more threads (or memory for one) to be had: those that run do the work
         }
         workers.store(started, std::memory_order_release);
         work(0, started);
