@@ -860,7 +860,7 @@ template <typename S> PairMap pair_map(const Handle *h, double *us)
         if (c <= 1.04 * best) pm.zc = (uint32_t)zc;
         best = std::min(best, c);
     }
-    if (const char *e = getenv("EUP_PAIR_ZC")) pm.zc = (uint32_t)atoi(e);
+    if (const char *e = getenv("EUP_PAIR_ZC")) pm.zc = (uint32_t)std::min(std::max(atoi(e), 1), g.n);
     pm.blocks = (uint32_t)(cols * ((g.n + (int)pm.zc - 1) / (int)pm.zc));
     pm.dnx = UDiv::make(pm.nx);
     pm.dny = UDiv::make(pm.ny);

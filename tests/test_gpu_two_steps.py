@@ -44,6 +44,20 @@ def test_two_steps_equal_single_steps(shape, x_open, storage, monkeypatch):
 
 
 @pytest.mark.parametrize("storage", ["f32", "f64"])
+@pytest.mark.parametrize("chunk", ["-3", "0", "100", ""])
+def test_chunk_switch_outside_the_lattice(chunk, storage, monkeypatch):
+    """The switch is held to 1 .. n planes."""
+    shape = (40, 16, 9)
+    print(f"two-step chunk switch {chunk!r} {storage}", flush=True)
+    mask = geometry.cylinder(*shape, 3, (12, 8))
+    one = after(shape, storage, True, mask, 4, "0", monkeypatch)
+    monkeypatch.setenv("EUP_PAIR_ZC", chunk)
+    two = after(shape, storage, True, mask, 4, "1", monkeypatch)
+    for a, b in zip(one, two):
+        assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("storage", ["f32", "f64"])
 @pytest.mark.parametrize("chunk", ["1", "3", "7"])
 def test_chunks_of_planes(chunk, storage, monkeypatch):
     """Any cut into chunks of planes gives the same state, the last chunk a short one."""
