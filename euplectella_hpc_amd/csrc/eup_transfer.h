@@ -5,7 +5,10 @@
 // 27 GB/s into warm and 14 GB/s into newly mapped memory, four 45 and 26, against the bus's 55; eight
 // threads were slower than four.  84 MB to newly mapped memory, measured: the runtime's copy of
 // pageable memory 8.0 ms in one call and 8.3 plane by plane, pinned pieces of 1 MB with one
-// thread 6.3, with four 3.3.
+// thread 6.3, with four 3.3.  To the device the bus is the limit (kernels read host memory at 36 GB/s, as
+// fast as the runtime's copy): fewer threads, which take less time to start, keep it busy up to 32 MB.  us
+// of the runtime's copy and with one, two and four threads: 3.1 MB 122, 111, 127, 123; 8.4 MB 262, 280,
+// 245, 265; 17 MB 485, 545, 460, 480; 84 MB (19 populations) 3700, 3400, 2050, 2000.
 #pragma once
 
 #include <string.h>
@@ -32,7 +35,8 @@ int transfer(Handle *h, char *host, int64_t bytes, int64_t unit, F &&launch)
 {
     const int64_t piece = bytes <= kMovePiece ? bytes : kMovePiece / unit * unit;
     const int64_t pieces = (bytes + piece - 1) / piece;
-    const int threads = (int)(pieces < kMoveThreads ? pieces : kMoveThreads);
+    const int most = !In || pieces >= 32 ? kMoveThreads : (pieces > 4 ? 2 : 1);
+    const int threads = (int)(pieces < most ? pieces : most);
     const int64_t slot = (piece + 4095) / 4096 * 4096;
     int rc = transfer_ready(h, slot * (pieces < kMoveSlots ? pieces : kMoveSlots));
     if (rc) return rc;
