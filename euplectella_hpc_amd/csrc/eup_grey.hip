@@ -600,39 +600,38 @@ template <typename R> int grey_step_t(Handle *h)
     return 0;
 }
 
-// the blocks' partial force sums, cleared, and three results after them
-int force_scratch(Handle *h, double **sum)
+// the blocks' partial force sums, cleared, and pinned memory for their total
+int force_scratch(Handle *h)
 {
-    const int64_t np = 3 * (int64_t)blocks_of(h->g.sites), len = np + 3;
-    if (h->diag_len < len) {
+    const int64_t np = 3 * (int64_t)blocks_of(h->g.sites);
+    if (pinned_ready(h, 3 * sizeof(double))) return EUP_EHIP;
+    if (h->diag_len < np) {
         hipFree(h->diag);
         h->diag = nullptr;
         h->diag_len = 0;
-        if (hip_check(h, hipMalloc((void **)&h->diag, sizeof(double) * len), "hipMalloc")) return EUP_EHIP;
-        h->diag_len = len;
+        if (hip_check(h, hipMalloc((void **)&h->diag, sizeof(double) * np), "hipMalloc")) return EUP_EHIP;
+        h->diag_len = np;
     }
     hipLaunchKernelGGL(k_fill0, dim3(blocks_of(np)), dim3(256), 0, h->stream, h->diag, np);
-    *sum = h->diag + np;
     return hip_check(h, hipGetLastError(), "force scratch") ? EUP_EHIP : 0;
 }
 
-int force_result(Handle *h, double *sum, double F[3])
+int force_result(Handle *h, double F[3])
 {
+    double *const sum = reinterpret_cast<double *>(h->pinned);
     hipLaunchKernelGGL(k_force_sum, dim3(1), dim3(1024), 0, h->stream, h->diag, (int)blocks_of(h->g.sites), sum);
-    if (hip_check(h, hipGetLastError(), "grey force") ||
-        hip_check(h, hipMemcpyAsync(F, sum, sizeof(double) * 3, hipMemcpyDeviceToHost, h->stream), "copy") ||
-        hip_check(h, hipStreamSynchronize(h->stream), "sync"))
+    if (hip_check(h, hipGetLastError(), "grey force") || hip_check(h, hipStreamSynchronize(h->stream), "sync"))
         return EUP_EHIP;
+    for (int c = 0; c < 3; ++c) F[c] = sum[c];
     return 0;
 }
 
 template <typename R> int grey_force_t(Handle *h, double F[3])
 {
-    double *sum;
-    if (int rc = force_scratch(h, &sum)) return rc;
+    if (int rc = force_scratch(h)) return rc;
     refresh_outlet<R>(h);
     launch_grey<R>(h, h->buf[h->cur], nullptr, 3);
-    return force_result(h, sum, F);
+    return force_result(h, F);
 }
 
 // A handle keeps its objective's device memory for the next call if it is at most this much
@@ -646,8 +645,7 @@ int objective_t(Handle *h, int t0, int t1, int K, double norm, double *J, void *
     const int64_t N = h->g.sites;
     const size_t S = (grey_state_bytes(h) + 255) / 256 * 256; // one state with its outlet plane
     const bool want_grad = grad_dev || grad_host;
-    double *sum;
-    if (int rc = force_scratch(h, &sum)) return rc;
+    if (int rc = force_scratch(h)) return rc;
     // Checkpoints: the states K, 2 K, ... up to t1 - 1, written by the forward sweep in place (state 0
     // is the handle's own).  A segment's other states, at most min(K, t1) - 1; the forward sweep leaves
     // those of the last segment there.  Two states for the rest of the forward sweep, the last one t1.
@@ -698,7 +696,7 @@ int objective_t(Handle *h, int t0, int t1, int K, double norm, double *J, void *
     for (int t = 0; t < t1; ++t) launch_grey<R>(h, state(t), state(t + 1), t >= t0 ? 1 : 0);
     launch_grey<R>(h, state(t1), nullptr, 1);
     double F[3];
-    if (int rc = force_result(h, sum, F)) return rc;
+    if (int rc = force_result(h, F)) return rc;
     const double wobj = 1.0 / ((double)(t1 - t0 + 1) * norm);
     *J = F[0] * wobj;
     if (!want_grad) return 0;
