@@ -58,6 +58,20 @@ def test_chunk_switch_outside_the_lattice(chunk, storage, monkeypatch):
 
 
 @pytest.mark.parametrize("storage", ["f32", "f64"])
+@pytest.mark.parametrize("x_open", [True, False])
+def test_more_workgroups_than_one_deal(x_open, storage, monkeypatch):
+    """Workgroups are dealt to the XCDs in whole groups of 256, the rest in order: 720 (FP32) and 1200 (FP64)."""
+    shape = (130, 66, 40)
+    print(f"two-step deal x_open={x_open} {storage}", flush=True)
+    mask = geometry.scattered(*shape, fraction=0.03, seed=5)
+    one = after(shape, storage, x_open, mask, 4, "0", monkeypatch)
+    monkeypatch.setenv("EUP_PAIR_ZC", "1")
+    two = after(shape, storage, x_open, mask, 4, "1", monkeypatch)
+    for a, b in zip(one, two):
+        assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("storage", ["f32", "f64"])
 @pytest.mark.parametrize("chunk", ["1", "3", "7"])
 def test_chunks_of_planes(chunk, storage, monkeypatch):
     """Any cut into chunks of planes gives the same state, the last chunk a short one."""
