@@ -191,7 +191,7 @@ __global__ __launch_bounds__(kBlock) void k_final(const double *partial, int nbl
 // momentum exchange over all interior sites (parity layout), neighbour test on the solid flags
 template <typename Acc>
 __global__ __launch_bounds__(kBlock) void k_mem_sites(Acc acc, const uint8_t *solid, int xopen,
-                                                      double *partial, uint32_t *ticket, double *out)
+                                                      double *partial)
 {
     const int l = acc.l, m = acc.m, n = acc.n;
     const int64_t N = (int64_t)l * m * n;
@@ -217,7 +217,7 @@ __global__ __launch_bounds__(kBlock) void k_mem_sites(Acc acc, const uint8_t *so
             v[2] += czs[p] * f2;
         }
     }
-    grid_reduce<3>(v, partial, ticket, out);
+    block_reduce<3>(v, partial);
 }
 
 // momentum exchange over the mixed tiles only (physics layout): bit opp(p) of the link mask of a
@@ -345,20 +345,20 @@ __global__ void k_vtk_vorticity(Acc acc, int k0, int64_t t0, int64_t count, floa
     out[o] = 0.5f * (mom[0] - mom[1]) - 0.5f * (mom[3] - mom[2]);
 }
 
-// I: unsigned type that holds the site numbers (divided twice per site; 32 bits where they suffice:
-// 192 x 768 x 768, e3m12, 1.63 -> 1.47 ms)
-template <typename Acc, typename I>
+// Site numbers in 32 bits (divided twice per site; in 64 bits 192 x 768 x 768, e3m12, took 1.63 ms, now
+// 1.47): a lattice has less than 2^31 sites, and the last stride past them fits as well.
+template <typename Acc>
 __global__ __launch_bounds__(kBlock) void k_diagno(Acc acc, const uint8_t *solid, double *partial)
 {
-    const I l = (I)acc.l, m = (I)acc.m;
-    const I N = l * m * (I)acc.n;
+    const uint32_t l = (uint32_t)acc.l, m = (uint32_t)acc.m;
+    const uint32_t N = l * m * (uint32_t)acc.n;
     double v[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-    for (I s = (I)blockIdx.x * kBlock + threadIdx.x; s < N; s += (I)gridDim.x * kBlock) {
+    for (uint32_t s = blockIdx.x * kBlock + threadIdx.x; s < N; s += gridDim.x * kBlock) {
         double rho, xj, yj, zj;
         if (solid[s]) {
             rho = 1.0; xj = 0.0; yj = 0.0; zj = 0.0;
         } else {
-            const I r = s / l, z = r / m;
+            const uint32_t r = s / l, z = r / m;
             const int i = 1 + (int)(s - r * l), j = 1 + (int)(r - z * m), k = 1 + (int)z;
             double x[19];
 #pragma unroll
@@ -607,7 +607,7 @@ int diag_drag_mem(Handle *h, double F[3])
         using A = decltype(acc);
         if constexpr (std::is_same_v<A, ParityAcc>) {
             hipLaunchKernelGGL((k_mem_sites<A>), dim3(blocks), dim3(kBlock), 0, h->stream, acc, h->solid, xopen,
-                               h->diag, ticket, res);
+                               h->diag);
         } else {
             using S = typename A::value_type;
             hipLaunchKernelGGL((k_mem_tiles<S>), dim3(blocks), dim3(kBlock), 0, h->stream, acc, h->mixed_list,
@@ -656,13 +656,7 @@ int diag_diagno(Handle *h, double out[5])
     double *tot = reinterpret_cast<double *>(h->pinned);
     rc = with_acc(h, [&](auto acc) {
         using A = decltype(acc);
-        // (the last stride may pass the last site: it has to fit as well)
-        if (h->g.sites < INT32_MAX)
-            hipLaunchKernelGGL((k_diagno<A, uint32_t>), dim3(kRedBlocks), dim3(kBlock), 0, h->stream, acc, h->solid,
-                               h->diag);
-        else
-            hipLaunchKernelGGL((k_diagno<A, uint64_t>), dim3(kRedBlocks), dim3(kBlock), 0, h->stream, acc, h->solid,
-                               h->diag);
+        hipLaunchKernelGGL((k_diagno<A>), dim3(kRedBlocks), dim3(kBlock), 0, h->stream, acc, h->solid, h->diag);
         return 0;
     });
     if (rc) return rc;
