@@ -560,10 +560,11 @@ template <typename R> GArgs<R> gargs(Handle *h, const void *from, void *to)
     return a;
 }
 
-// f(std::bool_constant<BIG>): arrays of 4 GiB and more take 64-bit offsets
+// f(std::bool_constant<BIG>): arrays of 4 GiB and more take 64-bit offsets (EUP_GREY_64BIT=1: all)
 template <typename R, typename F> void by_size(Handle *h, F &&f)
 {
-    if ((uint64_t)h->g.sites * sizeof(R) < (1ull << 32)) f(std::false_type{});
+    const char *e = getenv("EUP_GREY_64BIT");
+    if (!(e && atoi(e) != 0) && (uint64_t)h->g.sites * sizeof(R) < (1ull << 32)) f(std::false_type{});
     else f(std::true_type{});
 }
 

@@ -61,3 +61,28 @@ def test_steps_force_objective_and_gradient(shape, where, x_open):
         ref = dense(pops)
         orc.grey_steps(ref, s, om, U, 3, x_open=x_open)
         assert np.array_equal(dense(lat.get_state()), ref)
+
+
+@pytest.mark.parametrize("storage", ["f32", "f64"])
+@pytest.mark.parametrize("x_open", [True, False])
+@pytest.mark.parametrize("shape", [(70, 9, 5), (33, 7, 4)])
+def test_offsets_of_large_arrays_move_no_bit(shape, x_open, storage, monkeypatch):
+    """The kernels of arrays of 4 GiB and more, forced at a small size, against those of smaller ones."""
+    from euplectella_hpc_amd.lib import Lattice
+
+    print(f"grey offsets {shape} x_open={x_open} {storage}", flush=True)
+    got = []
+    for wide in ("0", "1"):
+        monkeypatch.setenv("EUP_GREY_64BIT", wide)
+        with Lattice(*shape, svisc=SVISC, u_inflow=U, mode="grey", storage=storage, x_open=x_open) as lat:
+            lat.set_grey(fields(*shape, "scattered"))
+            lat.init_equilibrium(U, 0.01, -0.02, 1e-3, 3)
+            lat.step(2)
+            F = lat.grey_force()
+            out = [F]
+            for fused in ("0", "1"):
+                monkeypatch.setenv("EUP_ADJ_FUSED", fused)
+                out += lat.grey_objective(2, 7, 3, 1.0)
+            got.append(out + [lat.get_state()])
+    for a, b in zip(*got):
+        assert np.array_equal(a, b)
