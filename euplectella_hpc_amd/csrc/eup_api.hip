@@ -320,8 +320,8 @@ int eup_set_mask(eup_handle *h, const int32_t *obs)
     if (hip_check(h, hipSetDevice(h->cfg.device), "hipSetDevice")) return EUP_EHIP;
     const Geometry &g = h->g;
     // validate values and build the dense solid flags on the host (setup-time work)
-    uint8_t *sol = nullptr;
-    if (hip_check(h, hipHostMalloc((void **)&sol, g.sites), "hipHostMalloc")) return EUP_EHIP;
+    const HostArray<uint8_t> sol(g.sites);
+    if (!sol.p) return fail(h, EUP_EHIP, "eup_set_mask: out of host memory");
     int64_t ns = 0;
     int bb[6] = {g.l, 0, g.m, 0, g.n, 0};
     for (int k = 1; k <= g.n; ++k)
@@ -329,10 +329,7 @@ int eup_set_mask(eup_handle *h, const int32_t *obs)
             for (int i = 1; i <= g.l; ++i) {
                 const int64_t o = (int64_t)(i - 1) + (int64_t)g.l * ((int64_t)(j - 1) + (int64_t)g.m * (k - 1));
                 const int32_t v = obs[o];
-                if (v != 0 && v != 1) {
-                    hipHostFree(sol);
-                    return fail(h, EUP_EINVAL, "eup_set_mask: obs values must be 0 or 1");
-                }
+                if (v != 0 && v != 1) return fail(h, EUP_EINVAL, "eup_set_mask: obs values must be 0 or 1");
                 sol[o] = (uint8_t)v;
                 if (v == 1) {
                     ++ns;
@@ -348,9 +345,8 @@ int eup_set_mask(eup_handle *h, const int32_t *obs)
     // (eup_step refuses it) rather than with tables that no longer match nsolid
     h->mask_set = false;
     int rc = 0;
-    if (hip_check(h, hipMemcpy(h->solid, sol, g.sites, hipMemcpyHostToDevice), "copy solid"))
+    if (hip_check(h, hipMemcpy(h->solid, sol.p, g.sites, hipMemcpyHostToDevice), "copy solid"))
         rc = EUP_EHIP;
-    hipHostFree(sol);
     if (rc) return rc;
     h->nsolid = ns;
     memcpy(h->bbox, bb, sizeof bb);

@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <stdlib.h>
 
 #include <string>
 
@@ -84,6 +85,17 @@ size_t occupancy_lds_bytes(const Handle *h, int cap);
 bool stream_stores(const Handle *h, double bytes);
 int hip_check(Handle *h, hipError_t e, const char *what);
 int pinned_ready(Handle *h, int64_t bytes); // h->pinned holds at least `bytes`
+
+// Host memory of one call's length.  Pageable: a pinned block that comes and goes costs up to 350 us
+// to allocate, depending on the sizes freed before it, and 20 to 100 us to free.
+template <typename T> struct HostArray {
+    T *p;
+    explicit HostArray(int64_t n) : p(static_cast<T *>(malloc(sizeof(T) * (size_t)(n > 0 ? n : 1)))) {}
+    ~HostArray() { free(p); }
+    HostArray(const HostArray &) = delete;
+    HostArray &operator=(const HostArray &) = delete;
+    T &operator[](int64_t i) const { return p[i]; }
+};
 
 // parity mode (eup_parity.hip)
 int parity_prepare_mask(Handle *h);

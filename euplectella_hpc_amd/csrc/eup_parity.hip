@@ -315,19 +315,13 @@ int parity_prepare_mask(Handle *h)
 {
     // solid list in the reference's bbox loop order (k, j, i), as offsets in the padded layout
     const Geometry &g = h->g;
-    uint8_t *sol_h = nullptr;
-    if (hip_check(h, hipHostMalloc((void **)&sol_h, g.sites), "hipHostMalloc")) return EUP_EHIP;
-    if (hip_check(h, hipMemcpy(sol_h, h->solid, g.sites, hipMemcpyDeviceToHost), "hipMemcpy solid")) {
-        hipHostFree(sol_h);
-        return EUP_EHIP;
-    }
+    const HostArray<uint8_t> sol_h(g.sites);
+    if (!sol_h.p) return fail(h, EUP_EHIP, "out of host memory for the solid flags");
+    if (hip_check(h, hipMemcpy(sol_h.p, h->solid, g.sites, hipMemcpyDeviceToHost), "hipMemcpy solid")) return EUP_EHIP;
     int64_t cnt = 0;
     for (int64_t s = 0; s < g.sites; ++s) cnt += sol_h[s] != 0;
-    int32_t *list_h = nullptr;
-    if (cnt > 0 && hip_check(h, hipHostMalloc((void **)&list_h, sizeof(int32_t) * cnt), "hipHostMalloc")) {
-        hipHostFree(sol_h);
-        return EUP_EHIP;
-    }
+    const HostArray<int32_t> list_h(cnt);
+    if (!list_h.p) return fail(h, EUP_EHIP, "out of host memory for the solid list");
     int64_t c = 0;
     for (int k = 1; k <= g.n; ++k)
         for (int j = 1; j <= g.m; ++j)
@@ -335,17 +329,15 @@ int parity_prepare_mask(Handle *h)
                 int64_t o = (int64_t)(i - 1) + (int64_t)g.l * ((int64_t)(j - 1) + (int64_t)g.m * (k - 1));
                 if (sol_h[o] != 0) list_h[c++] = (int32_t)parity_index(h, i, j, k);
             }
-    hipHostFree(sol_h);
     hipFree(h->solid_list);
     h->solid_list = nullptr;
     int rc = 0;
     if (cnt > 0) {
         if (hip_check(h, hipMalloc((void **)&h->solid_list, sizeof(int32_t) * cnt), "hipMalloc") ||
-            hip_check(h, hipMemcpy(h->solid_list, list_h, sizeof(int32_t) * cnt, hipMemcpyHostToDevice),
+            hip_check(h, hipMemcpy(h->solid_list, list_h.p, sizeof(int32_t) * cnt, hipMemcpyHostToDevice),
                       "hipMemcpy list"))
             rc = EUP_EHIP;
     }
-    if (list_h) hipHostFree(list_h);
     h->nsolid = cnt;
     return rc;
 }

@@ -1053,12 +1053,10 @@ int physics_prepare_mask(Handle *h)
                                (uint32_t)g.tiles);
             return hip_check(h, hipGetLastError(), "freeze") ? EUP_EHIP : 0;
         });
-    uint8_t *cls_h = nullptr;
-    int32_t *code_h = nullptr;
-    if (!rc && (hip_check(h, hipHostMalloc((void **)&cls_h, g.tiles), "hipHostMalloc") ||
-                hip_check(h, hipHostMalloc((void **)&code_h, sizeof(int32_t) * g.tiles), "hipHostMalloc")))
-        rc = EUP_EHIP;
-    if (!rc && hip_check(h, hipMemcpyAsync(cls_h, cls, g.tiles, hipMemcpyDeviceToHost, h->stream), "copy") )
+    const HostArray<uint8_t> cls_h(g.tiles);
+    const HostArray<int32_t> code_h(g.tiles), list_h(g.tiles);
+    if (!rc && !(cls_h.p && code_h.p && list_h.p)) rc = fail(h, EUP_EHIP, "out of host memory for the tile classes");
+    if (!rc && hip_check(h, hipMemcpyAsync(cls_h.p, cls, g.tiles, hipMemcpyDeviceToHost, h->stream), "copy") )
         rc = EUP_EHIP;
     if (!rc && hip_check(h, hipStreamSynchronize(h->stream), "sync")) rc = EUP_EHIP;
     int64_t nf = 0, nm = 0, ns = 0;
@@ -1078,7 +1076,7 @@ int physics_prepare_mask(Handle *h)
         if (hip_check(h, hipMalloc((void **)&h->tile_code, sizeof(int32_t) * g.tiles), "hipMalloc") ||
             hip_check(h, hipMalloc((void **)&h->link_mask, sizeof(uint32_t) * kTile * (nm + 2)),
                       "hipMalloc") ||
-            hip_check(h, hipMemcpyAsync(h->tile_code, code_h, sizeof(int32_t) * g.tiles,
+            hip_check(h, hipMemcpyAsync(h->tile_code, code_h.p, sizeof(int32_t) * g.tiles,
                                         hipMemcpyHostToDevice, h->stream), "copy"))
             rc = EUP_EHIP;
     }
@@ -1089,26 +1087,19 @@ int physics_prepare_mask(Handle *h)
     }
     if (!rc && nm > 0) {
         // mixed tile list for the momentum-exchange reduction
-        int32_t *list_h = nullptr;
-        if (hip_check(h, hipHostMalloc((void **)&list_h, sizeof(int32_t) * nm), "hipHostMalloc")) rc = EUP_EHIP;
-        if (!rc) {
-            for (int64_t t = 0; t < g.tiles; ++t)
-                if (code_h[t] >= 0) list_h[code_h[t]] = (int32_t)t;
-            hipFree(h->mixed_list);
-            h->mixed_list = nullptr;
-            if (hip_check(h, hipMalloc((void **)&h->mixed_list, sizeof(int32_t) * nm), "hipMalloc") ||
-                hip_check(h, hipMemcpyAsync(h->mixed_list, list_h, sizeof(int32_t) * nm,
-                                            hipMemcpyHostToDevice, h->stream), "copy"))
-                rc = EUP_EHIP;
-            if (!rc && hip_check(h, hipStreamSynchronize(h->stream), "sync")) rc = EUP_EHIP;
-            hipHostFree(list_h);
-        }
+        for (int64_t t = 0; t < g.tiles; ++t)
+            if (code_h[t] >= 0) list_h[code_h[t]] = (int32_t)t;
+        hipFree(h->mixed_list);
+        h->mixed_list = nullptr;
+        if (hip_check(h, hipMalloc((void **)&h->mixed_list, sizeof(int32_t) * nm), "hipMalloc") ||
+            hip_check(h, hipMemcpyAsync(h->mixed_list, list_h.p, sizeof(int32_t) * nm, hipMemcpyHostToDevice, h->stream),
+                      "copy"))
+            rc = EUP_EHIP;
     }
-    if (!rc && hip_check(h, hipStreamSynchronize(h->stream), "sync")) rc = EUP_EHIP;
+    // (also after an error: the copies read the arrays)
+    if (hip_check(h, hipStreamSynchronize(h->stream), "sync")) rc = EUP_EHIP;
     hipFree(cls);
     hipFree(link_all);
-    if (cls_h) hipHostFree(cls_h);
-    if (code_h) hipHostFree(code_h);
     h->outlet_dirty = true;
     return rc;
 }
