@@ -126,7 +126,8 @@ namespace eup {
 
 // Powers of two: the runtime keeps freed pinned blocks of these sizes and hands them out again (12 us, the
 // next handle's commit and transfers), where a block of 96 KB or 7 MB took 250 to 350 us each time,
-// the next 64 KB one too.  Creating a 128 x 64 x 64 parity lattice up to its start: 1.48 ms, now 1.07.
+// the next 64 KB one too.  Creating a 128 x 64 x 64 parity lattice up to its start: 1.48 ms before, 1.07
+// with these sizes (0.9 with the mask's host arrays pageable as well, HostArray).
 int pinned_ready(Handle *h, int64_t bytes)
 {
     if (h->pinned_len >= bytes) return 0;

@@ -27,13 +27,17 @@
 // the site x = l - 1 once more and put the outlet equilibrium of the result in place of the
 // populations that the second step pulls from there.
 //
-// Bound: memory.  Sponge 512 x 256 x 256 FP32: 0.567 ms per step against 0.831 ms in single steps, FP64
-// 1.27 against 1.66.  Without obstacles and with periodic x an FP32 step took 0.521 ms; 0.150 without
-// the kernel's loads and stores, 0.226 without the loads, 0.346 without the stores, 0.520 without the
-// collisions.  It read 3.4 GB and wrote 2.55 GB per two steps, 5.7 TB/s: the extra reads are the halo
-// (15 / 13 rows, 34 / 32 planes and the lines that cut the columns).  The 2-byte storages do not gain
-// (their conversions add a half to the arithmetic while the bytes halve: FP16 0.424 against 0.419 ms)
-// and stay with single steps.
+// Bound: memory, short of a copy's 6.2 TB/s.  Sponge 512 x 256 x 256 FP32: 0.57 to 0.61 ms per step
+// between boxes against 0.82 to 0.83 in single steps, for 2.95 GB (5.1 TB/s at 0.58 ms); FP64 1.27 ms
+// against 1.66, 6.21 GB (4.9 TB/s).  Without obstacles 0.569 ms with open and 0.52 to 0.53 with periodic
+// x (FP32); the latter took 0.150 without the kernel's loads and stores, 0.226 without the loads, 0.346
+// without the stores, 0.520 without the collisions.  It read 3.4 GB and wrote 2.55 GB per two steps,
+// 5.7 TB/s: the extra reads are the halo (15 / 13 rows, 34 / 32 planes and the lines that cut the columns).
+// What keeps it below the copy rate: one workgroup per CU (its LDS), whose wavefronts meet at two barriers
+// per plane.  The 2-byte storages stay with single steps: a form of this kernel for FP16 took 0.424
+// against 0.418 ms with open x and 0.470 against 0.427 on the sponge, though 0.374 against 0.418 with
+// periodic x.  What bounds that form is not known: neither its arithmetic (about 0.23 ms with the
+// conversions) nor its bytes (0.26) come to as much.
 #pragma once
 
 template <typename S> struct PairShape; // inner sites of a window

@@ -779,9 +779,9 @@ static size_t fused_lds_bytes(const Handle *h) { return occupancy_lds_bytes(h, f
 
 } // namespace
 
-// Whether a step's stores go past the caches (non-temporal).  They do not where the two state buffers
-// stay in the 256 MB memory-side cache from step to step, down to the 32 MB of the L2 caches.  us per
-// step, non-temporal against cached, without obstacles (MB of the two buffers): FP64 128 x 64 x 64 (159)
+// Whether a step's stores go past the caches (non-temporal).  They do not between 50 and 280 MB of state
+// buffers, where what a step stored is still found in the caches (mostly the 256 MB memory-side one) by
+// the next; both limits are where the measured times cross.  us per step, non-temporal against cached, without obstacles (MB of the two buffers): FP64 128 x 64 x 64 (159)
 // 30.3 / 25.7, 128 x 128 x 64 (319) 55.3 / 56.7, 192 x 96 x 96 (538) 89.7 / 99.2; FP32 64 x 64 x 64
 // (40) 8.4 / 9.3, 128 x 64 x 64 (80) 16.3 / 14.1, 192 x 96 x 96 (269) 47.2 / 43.0 (two steps per launch
 // 39.1 / 36.6), 256 x 128 x 64 (319) 54.8 / 53.8 (44.8 / 46.5); FP16 256 x 128 x 64 (159) 29.1 / 26.9, 256 x

@@ -111,7 +111,8 @@ const char *eup_last_error(const eup_handle *h);
 /* --- state --------------------------------------------------------------------------------- */
 
 /* Solid mask obs(1:l,1:m,1:n), int32, i fastest, 1 = solid -- the array build_obs fills
- * (build.obs.F90:147-186).  Computes the obstacle bounding box and the tile classes. */
+ * (build.obs.F90:147-186).  Computes the obstacle bounding box and the tile classes.  Between steps a
+ * new mask may be set: in physics mode a site that becomes solid keeps the populations it has then. */
 int eup_set_mask(eup_handle *h, const int32_t *obs);
 
 /* The obstacle list itself, streamed in chunks, without a dense host array: the file
@@ -229,7 +230,10 @@ int eup_grey_force(eup_handle *h, double F[3]);
 
 /* J = sum_{t=t0..t1} F_x(a^t) / ((t1 - t0 + 1) * norm), a^0 = the current state (left unchanged),
  * and, if grad is not NULL, dJ/ds(1:l,1:m,1:n) by the discrete adjoint; forward states are
- * checkpointed every `every` steps and recomputed per segment.  Host FP64 gradient. */
+ * checkpointed every `every` steps and recomputed per segment.  Host FP64 gradient.  The device
+ * memory of a call, (t1 - 1) / every + min(every, t1) + 4 states and 8 bytes per site (2 states
+ * without grad), stays with the handle for the next call if it is at most 2 GiB, until
+ * eup_destroy; more is freed when the call returns. */
 int eup_grey_objective(eup_handle *h, int32_t t0, int32_t t1, int32_t every, double norm, double *J,
                        double *grad);
 
